@@ -315,14 +315,25 @@ int cols_per_launch(const TileGeom &g, size_t max_lds) {
 constexpr size_t kPrefillMinCols = 32;
 constexpr size_t kFastMinCols = 64;
 
+// What the matrix-core kernels can take of a launch's weights: `tiles` all of
+// them (the tiles they address, below), `f16` also as single f16 operands (no
+// Q6_K weight with scales beyond those, Handle::f16_exact).
+struct MfmaFit {
+  bool tiles, f16;
+};
+
 // 0: not a prefill launch, 1: bit-exact prefill, 2: fast prefill
-// f16ok: the matrix-core kernels can take every weight of the launch
-// (mfma_ok: exact f16 operands, tiles they can address); otherwise no prefill
-// kernel applies, forced or not.
-int prefill_kind(size_t cols, bool f16ok) {
+// The automatic fast kernel takes every Q6_K weight (with full-range scales
+// as two exact operands, MfmaLaunch::wide6); the other prefill kernels, and
+// the forced fast one, take launches with single f16 operands only.
+int prefill_kind(size_t cols, MfmaFit fit) {
   const State &s = st();
   const int forced = s.matvec_kernel;
-  if (!f16ok) return 0;
+  if (!fit.tiles) return 0;
+  if (!fit.f16) {
+    const bool fast = forced == 0 && cols >= kFastMinCols && !s.host_exact && prefill_fast_lds_bytes() <= s.max_lds;
+    return fast ? 2 : 0;
+  }
   const bool exact_fits = prefill_lds_bytes() <= s.max_lds;
   const bool fast_fits = prefill_fast_lds_bytes() <= s.max_lds;
   if (forced == 4) return exact_fits ? 1 : 0;
@@ -375,16 +386,18 @@ int wide_rows_for(int rows, int nb, int cols, int type) {
 
 int g_nb_of(Handle *const *hs) { return hs[0]->g.nb; }
 
-// The matrix-core kernels can take these weights: their f16 operands are
-// exact, and when the launch reads its weights from their tiles (one of them
-// kept without segments makes every weight of the launch read that way),
-// each fits the kernels' 32-bit tile offsets (under 4 GiB).
-bool mfma_ok(size_t count, Handle *const *hs) {
+// When a launch reads its weights from their tiles (one of them kept without
+// segments makes every weight of the launch read that way), each must fit the
+// matrix-core kernels' 32-bit tile offsets (under 4 GiB).
+MfmaFit mfma_fit(size_t count, Handle *const *hs) {
   bool tiles = false;
+  MfmaFit f{true, true};
   for (size_t i = 0; i < count; i++) tiles = tiles || !hs[i]->segs;
-  for (size_t i = 0; i < count; i++)
-    if (!hs[i]->f16_exact || (tiles && hs[i]->byte_length >= ((size_t)1 << 32))) return false;
-  return true;
+  for (size_t i = 0; i < count; i++) {
+    if (tiles && hs[i]->byte_length >= ((size_t)1 << 32)) f = MfmaFit{false, false};
+    if (!hs[i]->f16_exact) f.f16 = false;
+  }
+  return f;
 }
 
 bool use_wide(size_t count, Handle *const *hs, size_t cols) {
@@ -447,21 +460,21 @@ int32_t run_norm(const float *y, int rows, int n, const float *w_post, const flo
 // Whether a one-column launch over these weights runs a vector-ALU kernel,
 // which can form its input with the norm prologue.
 bool norm_prologue_ok(size_t count, Handle *const *hs, size_t cols) {
-  const bool f16 = mfma_ok(count, hs);
-  if (cols != 1 || hs[0]->g.nb > 16 || prefill_kind(cols, f16) != 0) return false;
+  const MfmaFit fit = mfma_fit(count, hs);
+  if (cols != 1 || hs[0]->g.nb > 16 || prefill_kind(cols, fit) != 0) return false;
   int tiles16 = 0;
   for (size_t i = 0; i < count; i++) tiles16 += (int)((hs[i]->row_count + 15) / 16);
-  return !use_mfma(cols, hs[0]->g.nb, tiles16, f16);
+  return !use_mfma(cols, hs[0]->g.nb, tiles16, fit.f16);
 }
 
 // Whether a launch of `cols` columns (2 or more) runs the vector-ALU kernels
 // in one chunk, so it can take its input as a pre-quantised image.
 bool image_input_ok(size_t count, Handle *const *hs, size_t cols) {
-  const bool f16 = mfma_ok(count, hs);
-  if (cols < 2 || prefill_kind(cols, f16) != 0) return false;
+  const MfmaFit fit = mfma_fit(count, hs);
+  if (cols < 2 || prefill_kind(cols, fit) != 0) return false;
   int tiles16 = 0;
   for (size_t i = 0; i < count; i++) tiles16 += (int)((hs[i]->row_count + 15) / 16);
-  return !use_mfma(cols, hs[0]->g.nb, tiles16, f16) && cols_per_launch(hs[0]->g, st().max_lds) >= (int)cols;
+  return !use_mfma(cols, hs[0]->g.nb, tiles16, fit.f16) && cols_per_launch(hs[0]->g, st().max_lds) >= (int)cols;
 }
 
 // norm != null: the input is formed from a residual stream (NormIn) -- in the
@@ -481,10 +494,10 @@ int32_t run_matvec(size_t count, Handle *const *hs, const float *d_input, size_t
   if (cols == 0) return HP_OK;
   if (tail_in && !tail_in->part) tail_in = nullptr;
   const bool image_ok = s.images && cols >= 2 && image_input_ok(count, hs, cols);
-  const bool f16 = mfma_ok(count, hs);
-  const bool wide = prefill_kind(cols, f16) == 0 && use_wide(count, hs, cols);
+  const MfmaFit fit = mfma_fit(count, hs);
+  const bool wide = prefill_kind(cols, fit) == 0 && use_wide(count, hs, cols);
   const bool wide_norm = wide && cols == 1 && g_nb_of(hs) <= 16;  // the wide kernel's norm prologue
-  const int kind = prefill_kind(cols, f16);
+  const int kind = prefill_kind(cols, fit);
   if (kind && cols > 65535) return fail(HP_ERR_SHAPE, "too many columns");
   // a deferred GeGLU tail is completed by the fast prefill kernel's pre-pass
   if (tail_in && (kind != 2 || norm || tiles_in)) return fail(HP_ERR_ARG, "deferred GeGLU tail needs the fast prefill");
@@ -502,6 +515,7 @@ int32_t run_matvec(size_t count, Handle *const *hs, const float *d_input, size_t
     l.rows[i] = (int)hs[i]->row_count;
     l.out[i] = d_outs[i];
   }
+  l.wide6 = !fit.f16;
   uint8_t *pre = nullptr;  // the prefill kernels' scratch
   if (kind) {
     const size_t need = kind == 2 ? prefill_fast_bytes(l, s.num_cus) : prefill_q8k_bytes((int)input_size, (int)cols);
@@ -595,7 +609,7 @@ int32_t run_matvec(size_t count, Handle *const *hs, const float *d_input, size_t
   }
   int tiles16 = 0;
   for (size_t i = 0; i < count; i++) tiles16 += (int)((hs[i]->row_count + 15) / 16);
-  if (use_mfma(cols, g.nb, tiles16, f16)) {
+  if (use_mfma(cols, g.nb, tiles16, fit.f16)) {
     MfmaLaunch l{};
     l.count = (int)count;
     l.k = (int)input_size;
@@ -664,12 +678,12 @@ int32_t run_matvec_geglu(Handle *hg, Handle *hu, const float *d_input, size_t in
   const TileGeom g = hg->g;
   const int tiles16 = 2 * (int)((rows + 15) / 16);
   Handle *pair[2] = {hg, hu};
-  const bool f16 = mfma_ok(2, pair);
-  const bool wide = prefill_kind(cols, f16) == 0 && hg->type == hu->type && use_wide_pair(pair, cols);
-  const bool fused = !wide && cols <= 4 && s.matvec_kernel <= 1 && !use_mfma(cols, g.nb, tiles16, f16) &&
+  const MfmaFit fit = mfma_fit(2, pair);
+  const bool wide = prefill_kind(cols, fit) == 0 && hg->type == hu->type && use_wide_pair(pair, cols);
+  const bool fused = !wide && cols <= 4 && s.matvec_kernel <= 1 && !use_mfma(cols, g.nb, tiles16, fit.f16) &&
                      !use_half((int)cols, g, 2 * hg->tiles, (int)(2 * rows)) && cols_per_launch(g, s.max_lds) >= (int)cols;
   // fast prefill: gate and up rows in one tile, GeGLU in its epilogue
-  const bool fast = prefill_kind(cols, f16) == 2 && hg->type == hu->type;
+  const bool fast = prefill_kind(cols, fit) == 2 && hg->type == hu->type;
   MfmaLaunch l{};
   uint8_t *pre = nullptr;  // its scratch, tiles first
   if (fast) {
@@ -685,6 +699,7 @@ int32_t run_matvec_geglu(Handle *hg, Handle *hu, const float *d_input, size_t in
       l.type[i] = pair[i]->type;
       l.rows[i] = (int)rows;
     }
+    l.wide6 = !fit.f16;
     void *p = nullptr;
     int32_t rc = stream_scratch(stream, kScratchPrefill, prefill_fast_geglu_bytes(l, s.num_cus), &p);
     if (rc != HP_OK) return rc;
@@ -2554,7 +2569,7 @@ int32_t hp_hip_decode_layers_device(const hp_hip_decode_layer_t *layers, size_t 
         // O on the fast prefill kernel: the slice merge writes its
         // activation tiles into O's prefill scratch (the pre-pass launch
         // they replace would write the same bytes there)
-        if (s.prefill_folds && prefill_kind(Mc, mfma_ok(1, &H.o)) == 2 && H.o->input_size % kQK == 0 &&
+        if (s.prefill_folds && prefill_kind(Mc, mfma_fit(1, &H.o)) == 2 && H.o->input_size % kQK == 0 &&
             H.o->input_size == (size_t)L.attention.head_count * kHeadDim) {
           MfmaLaunch lo{};
           lo.count = 1;
@@ -2593,7 +2608,7 @@ int32_t hp_hip_decode_layers_device(const hp_hip_decode_layer_t *layers, size_t 
       // down on the fast prefill kernel: its pre-pass completes the gate/up
       // launch's trailing tiles (no tail launch)
       Handle *dh[1] = {H.down};
-      const bool down_fast = s.prefill_folds && prefill_kind(Mc, mfma_ok(1, dh)) == 2 && H.down->input_size % kQK == 0;
+      const bool down_fast = s.prefill_folds && prefill_kind(Mc, mfma_fit(1, dh)) == 2 && H.down->input_size % kQK == 0;
       GegluTail gtail{};
       rc = run_matvec_geglu(H.gate, H.up, nullptr, hidden, Mc, h, strm, &fin, xn, imgh, &h_img, &op,
                             down_fast ? &gtail : nullptr);

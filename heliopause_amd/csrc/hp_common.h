@@ -401,6 +401,7 @@ struct MfmaLaunch {
   int k;
   int cols;        // 1..8 columns in this launch
   int out_col0;
+  bool wide6;      // some Q6_K weight's sc * (q - 32) is inexact in one f16 (two-part fragments)
 };
 size_t mfma_segment_bytes(int type, int rows, int nb);
 size_t mfma_lds_bytes(int cols, int nb);

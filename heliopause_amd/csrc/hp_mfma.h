@@ -73,14 +73,41 @@ __device__ __forceinline__ half2v dup_byte_16th(uint32_t v, int idx) {
   return h - (half2v){(_Float16)64.0f, (_Float16)64.0f};
 }
 
+__device__ __forceinline__ half8 cat(half2v a, half2v b, half2v c, half2v d) {
+  return (half8){a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
+}
+
+// Q6_K with any int8 scale: sc * (q - 32) reaches 4096 in magnitude, and f16
+// holds integers beyond 2048 only when even, so it enters as two exact parts,
+// (sc & ~1) * (q - 32) (even) and (sc & 1) * (q - 32), each its own MFMA on
+// the same accumulator.  Every partial sum over one class stays an integer of
+// at most 2^24: 32 x 32 x 128 x 128, and the odd parts only shrink the terms
+// of negative odd scales (127 = 128 - 1) and complete the positive ones.
+// Scales of a 4-byte group word as even parts (s0, s1), (s2, s3) and odd masks.
+__device__ __forceinline__ void q6_split_scales(half2v (&S)[2], uint32_t (&M)[2], uint32_t gs) {
+  const uint32_t u = gs ^ 0x80808080u;  // s + 128 (128 is even: same parity)
+  const half2v b1152 = (half2v){(_Float16)1152.0f, (_Float16)1152.0f};
+  S[0] = magic_pair<kSel01>(u & 0xFEFEFEFEu) - b1152;
+  S[1] = magic_pair<kSel23>(u & 0xFEFEFEFEu) - b1152;
+  const uint32_t o = (u & 0x01010101u) * 0xFFu;  // 0xFF per odd byte
+  M[0] = __builtin_amdgcn_perm(0u, o, 0x01010000u);
+  M[1] = __builtin_amdgcn_perm(0u, o, 0x03030202u);
+}
+// Two dwords of 6-bit values (bytes 0, 2, 1, 3 of lo, then of hi) times their
+// scales, as the two parts.
+__device__ __forceinline__ void q6_split(half8 &even, half8 &odd, uint32_t lo, uint32_t hi, const half2v (&S)[2],
+                                         const uint32_t (&M)[2]) {
+  const half2v b1056 = (half2v){(_Float16)1056.0f, (_Float16)1056.0f};  // 1024 + 32
+  const half2v a = magic_pair<kSel02>(lo) - b1056, b = magic_pair<kSel13>(lo) - b1056;
+  const half2v c = magic_pair<kSel02>(hi) - b1056, d = magic_pair<kSel13>(hi) - b1056;
+  even = cat(a * S[0], b * S[0], c * S[1], d * S[1]);
+  odd = cat(as_h2(as_u32(a) & M[0]), as_h2(as_u32(b) & M[0]), as_h2(as_u32(c) & M[1]), as_h2(as_u32(d) & M[1]));
+}
+
 __device__ __forceinline__ half2v fma2(half2v a, half2v b, half2v c) { return __builtin_elementwise_fma(a, b, c); }
 
 __device__ __forceinline__ f32x4 mfma(half8 a, half8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-}
-
-__device__ __forceinline__ half8 cat(half2v a, half2v b, half2v c, half2v d) {
-  return (half8){a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
 }
 
 }  // namespace hp

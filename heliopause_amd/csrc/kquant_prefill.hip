@@ -631,12 +631,31 @@ __device__ __forceinline__ half8 f3_a(const typename WSel<Q4>::T &w, const uint3
   }
 }
 
+// Q6_K weights whose scales reach beyond what one f16 holds exactly (an odd
+// scale of 67 and more against an odd q - 32; hp_mfma.h): the fragment as two
+// exact ones, (sc & ~1) * (q - 32), at most 4096 and even, and (sc & 1) *
+// (q - 32).  S are the even parts (pairs as f3_a's), M the odd bits as masks.
+// Costs twice the MFMAs and 8 more vector-ALU instructions per fragment; the
+// vector-ALU kernels these weights took before re-read them every 8 columns:
+// three layers over 512 tokens 14.65 -> 0.88 ms, over 150 tokens 4.42 -> 0.44.
+template <bool TILE>
+__device__ __forceinline__ void f3_a6_split(half8 &hi8, half8 &lo8, const W6 &w, const uint32_t (&qd)[2][4], int l,
+                                            int q, const half2v (&S)[2], const uint32_t (&M)[2]) {
+  const int g = l & 1, t = l >> 1, jj = 2 * (q & 1);
+  const uint32_t ql = qd[g][t], qh = u4at(w.qh[t >> 1], 2 * (t & 1) + g) ^ (TILE ? 0xAAAAAAAAu : 0u);
+  const uint32_t lo = (ql & 0x0F0F0F0Fu) | (((qh >> (2 * jj)) & 0x03030303u) << 4);
+  const uint32_t hi = ((ql >> 4) & 0x0F0F0F0Fu) | (((qh >> (2 * jj + 2)) & 0x03030303u) << 4);
+  q6_split(hi8, lo8, lo, hi, S, M);
+}
+
 // One block of the wave's tile (kF3RS segments x 64 columns): weights w
 // against the activation tile at xl.  Segments past the weight's end repeat
-// the last one and are never stored.
-template <bool Q4, bool TILE>
+// the last one and are never stored.  X6: Q6_K fragments as two exact parts
+// (f3_a6_split), two MFMAs each.
+template <bool Q4, bool TILE, bool X6>
 __device__ __forceinline__ void f3_block(float (&out)[kF3RS][kF3CS][4], const typename WSel<Q4>::T (&w)[kF3RS],
                                          const uint8_t *xl, int lane, uint32_t exp) {
+  constexpr bool SPLIT = X6 && !Q4;
   // Wave priority: the block's set-up and class loop (the matrix cores'
   // work) issue ahead of the other wave of the SIMD while that one runs its
   // f32 tail, which lowers it again below: the MFMA pipe stays fed through
@@ -647,6 +666,7 @@ __device__ __forceinline__ void f3_block(float (&out)[kF3RS][kF3CS][4], const ty
   // column set cs: 16-column slice cs % 4 of activation tile cs / 4
   auto xh = [&](int cs) { return reinterpret_cast<const _Float16 *>(xl + (cs >> 2) * kF2XTile); };
   half2v S[kF3RS][2], N[kF3RS][2];
+  uint32_t odd[kF3RS][2];  // SPLIT: the odd bits of the scales, as masks
 #pragma unroll
   for (int rs = 0; rs < kF3RS; rs++) {
     if constexpr (Q4) {
@@ -659,6 +679,8 @@ __device__ __forceinline__ void f3_block(float (&out)[kF3RS][kF3CS][4], const ty
       const half2v m1024 = (half2v){(_Float16)-1024.0f, (_Float16)-1024.0f};
 #pragma unroll
       for (int e = 0; e < 2; e++) N[rs][e] = S[rs][e] * m1024;
+    } else if constexpr (SPLIT) {
+      q6_split_scales(S[rs], odd[rs], w[rs].gs);
     } else {
       // signed scales: bytes ^ 0x80 are s + 128; (1024 + 128 + s) - 1152 = s
       const uint32_t gs = w[rs].gs ^ 0x80808080u;
@@ -696,31 +718,46 @@ __device__ __forceinline__ void f3_block(float (&out)[kF3RS][kF3CS][4], const ty
   for (int cs = 0; cs < kF3CS; cs++)
     B[0][cs] = __builtin_bit_cast(half8,
                                   *reinterpret_cast<const uint4 *>(xh(cs) + (q * kF2Cols + 16 * (cs & 3) + n) * 8));
-  half8 An[kF3RS];
+  half8 An[kF3RS], Ln[kF3RS];  // (Ln: the odd-scale part, SPLIT only)
+  auto unpack = [&](int rs, int l) {
+    if constexpr (SPLIT)
+      f3_a6_split<TILE>(An[rs], Ln[rs], w[rs], qd[rs], l, q, S[rs], odd[rs]);
+    else
+      An[rs] = f3_a<Q4, TILE>(w[rs], qd[rs], l, q, S[rs], N[rs], exp);
+  };
 #pragma unroll
-  for (int rs = 0; rs < kF3RS; rs++) An[rs] = f3_a<Q4, TILE>(w[rs], qd[rs], 0, q, S[rs], N[rs], exp);
+  for (int rs = 0; rs < kF3RS; rs++) unpack(rs, 0);
 #pragma unroll
   for (int l = 0; l < 8; l++) {
-    half8 A[kF3RS];
+    half8 A[kF3RS], Al[kF3RS];
 #pragma unroll
-    for (int rs = 0; rs < kF3RS; rs++) A[rs] = An[rs];
+    for (int rs = 0; rs < kF3RS; rs++) {
+      A[rs] = An[rs];
+      if constexpr (SPLIT) Al[rs] = Ln[rs];
+    }
     if (l < 7) {
 #pragma unroll
       for (int cs = 0; cs < kF3CS; cs++)
         B[(l + 1) & 1][cs] = __builtin_bit_cast(
             half8, *reinterpret_cast<const uint4 *>(xh(cs) + (((l + 1) * 4 + q) * kF2Cols + 16 * (cs & 3) + n) * 8));
 #pragma unroll
-      for (int rs = 0; rs < kF3RS; rs++) An[rs] = f3_a<Q4, TILE>(w[rs], qd[rs], l + 1, q, S[rs], N[rs], exp);
+      for (int rs = 0; rs < kF3RS; rs++) unpack(rs, l + 1);
     }
 #pragma unroll
     for (int cs = 0; cs < kF3CS; cs++)
 #pragma unroll
       for (int rs = 0; rs < kF3RS; rs++)
         D[rs][cs] = mfma(B[l & 1][cs], A[rs], l == 0 ? (f32x4){0.0f, 0.0f, 0.0f, 0.0f} : D[rs][cs]);
+    if constexpr (SPLIT) {
+#pragma unroll
+      for (int cs = 0; cs < kF3CS; cs++)
+#pragma unroll
+        for (int rs = 0; rs < kF3RS; rs++) D[rs][cs] = mfma(B[l & 1][cs], Al[rs], D[rs][cs]);
+    }
     if (l < 7) {
       __builtin_amdgcn_sched_group_barrier(0x100, kF3CS, 0);  // the B reads first
 #pragma unroll
-      for (int k = 0; k < kF3CS * kF3RS; k++) {
+      for (int k = 0; k < kF3CS * kF3RS * (SPLIT ? 2 : 1); k++) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
         __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);  // up to 3 vector-ALU
       }
@@ -839,7 +876,7 @@ __device__ __forceinline__ void f3_xcopy(const uint8_t *const (&xt)[kF3Tiles], i
 // tiles.  Loads are unconditional (the block index is clamped), so they never
 // sit behind a branch; every copy has landed (vmcnt(0)) before the barrier
 // that ends its block.
-template <bool Q4, bool TILE>
+template <bool Q4, bool TILE, bool X6>
 __device__ __forceinline__ void f3_tile(float (&out)[kF3RS][kF3CS][4], const PfWeight &W, int nb, int S, int R,
                                         int s0, const uint8_t *const (&xt)[kF3Tiles], int b0, int b1) {
   if (b1 <= b0) return;  // (block ranges hold at least two blocks)
@@ -862,7 +899,7 @@ __device__ __forceinline__ void f3_tile(float (&out)[kF3RS][kF3CS][4], const PfW
     f3_xcopy(xt, bn, f3_st1, wave, lane);
     f3_wloads<Q4, TILE>(wb, W, f, s0, bn, S, lane);
     __builtin_amdgcn_sched_barrier(0);  // the loads stay ahead of the block's compute
-    f3_block<Q4, TILE>(out, wa, f3_st0, lane, exp);
+    f3_block<Q4, TILE, X6>(out, wa, f3_st0, lane, exp);
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     if (b + 1 >= b1) break;
@@ -870,7 +907,7 @@ __device__ __forceinline__ void f3_tile(float (&out)[kF3RS][kF3CS][4], const PfW
     f3_xcopy(xt, bn2, f3_st0, wave, lane);
     f3_wloads<Q4, TILE>(wa, W, f, s0, bn2, S, lane);
     __builtin_amdgcn_sched_barrier(0);
-    f3_block<Q4, TILE>(out, wb, f3_st1, lane, exp);
+    f3_block<Q4, TILE, X6>(out, wb, f3_st1, lane, exp);
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     if (b + 2 >= b1) break;
@@ -895,8 +932,10 @@ constexpr int kF3WaveFloats = kF3RS * kF3CS * 4 * 64;  // a wave's sums (out) of
 // through LDS to the gate wave of the same rows, which stores
 // fround(gelu(gate) * up).  total_rt then counts those tiles, ksplit is 1.
 // TILE: every weight is read from its tiles (a launch with a weight kept in
-// one layout); else from its segments.
-template <bool PAIR, bool TILE>
+// one layout); else from its segments.  X6: some Q6_K weight's scales need
+// the two-part fragments (f3_a6_split); every Q6_K weight of the launch then
+// takes them (the same integers either way).
+template <bool PAIR, bool TILE, bool X6>
 __global__ __launch_bounds__(kF3Threads) __attribute__((amdgpu_waves_per_eu(kF3PerSIMD, kF3PerSIMD))) void
 kquant_prefill_fast_kernel(
     const F2Args a) {
@@ -948,9 +987,9 @@ kquant_prefill_fast_kernel(
 #pragma unroll
     for (int t = 0; t < kF3Tiles; t++) xt[t] = a.xt + (size_t)min(ct * kF3Tiles + t, xtiles - 1) * a.nb * kF2XTile;
     if (W.type == kTypeQ4K)
-      f3_tile<true, TILE>(out, WW, a.nb, a.S, a.R, T0 + my_seg, xt, b_begin, b_end);
+      f3_tile<true, TILE, X6>(out, WW, a.nb, a.S, a.R, T0 + my_seg, xt, b_begin, b_end);
     else
-      f3_tile<false, TILE>(out, WW, a.nb, a.S, a.R, T0 + my_seg, xt, b_begin, b_end);
+      f3_tile<false, TILE, X6>(out, WW, a.nb, a.S, a.R, T0 + my_seg, xt, b_begin, b_end);
     const int n = lane & 15, q = lane >> 4;
     if (PAIR && split) {
       float *part = a.tail_part + ((size_t)hidx * kF3Waves + wave) * kF3WaveFloats + lane;
@@ -1003,6 +1042,14 @@ kquant_prefill_fast_kernel(
       }
     }
   }
+}
+
+template <bool PAIR>
+void launch_fast_kernel(const F2Args &a, bool tiles, bool wide6, int grid, hipStream_t s) {
+  auto *k = tiles ? (wide6 ? kquant_prefill_fast_kernel<PAIR, true, true> : kquant_prefill_fast_kernel<PAIR, true, false>)
+                  : (wide6 ? kquant_prefill_fast_kernel<PAIR, false, true>
+                           : kquant_prefill_fast_kernel<PAIR, false, false>);
+  hipLaunchKernelGGL(k, dim3(grid), dim3(kF3Threads), 0, s, a);
 }
 
 // The gate/up items run as two block ranges (a.tail_full on): gate = range 0
@@ -1239,10 +1286,7 @@ hipError_t launch_prefill_fast_geglu(const MfmaLaunch &l, const float *x, uint8_
   a.tail_full = p.tail_full;
   a.tail_part = defer && tail_part ? tail_part : reinterpret_cast<float *>(scratch + (size_t)p.xtiles * nb * kF2XTile);
   if (defer) *defer = GegluTail{};
-  if (launch_reads_tiles(l))
-    hipLaunchKernelGGL((kquant_prefill_fast_kernel<true, true>), dim3(p.grid), dim3(kF3Threads), 0, s, a);
-  else
-    hipLaunchKernelGGL((kquant_prefill_fast_kernel<true, false>), dim3(p.grid), dim3(kF3Threads), 0, s, a);
+  launch_fast_kernel<true>(a, launch_reads_tiles(l), l.wide6, p.grid, s);
   if (!p.tail_full) return hipGetLastError();
   e = hipGetLastError();
   if (e != hipSuccess) return e;
@@ -1328,10 +1372,7 @@ hipError_t launch_prefill_fast(const MfmaLaunch &l, const float *x, uint8_t *scr
   }
   const long long items = (long long)a.total_rt * a.col_tiles * a.ksplit;
   const int grid = (int)(items < kF3PerCU * num_cus ? items : kF3PerCU * num_cus);
-  if (launch_reads_tiles(l))
-    hipLaunchKernelGGL((kquant_prefill_fast_kernel<false, true>), dim3(grid), dim3(kF3Threads), 0, s, a);
-  else
-    hipLaunchKernelGGL((kquant_prefill_fast_kernel<false, false>), dim3(grid), dim3(kF3Threads), 0, s, a);
+  launch_fast_kernel<false>(a, launch_reads_tiles(l), l.wide6, grid, s);
   if (a.ksplit == 1 || deferred) return hipGetLastError();
   e = hipGetLastError();
   if (e != hipSuccess) return e;
