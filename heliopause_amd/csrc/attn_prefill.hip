@@ -402,7 +402,7 @@ __global__ __launch_bounds__(256) void attn_merge_slices_kernel(const AttnArgs a
         v[4 * c + 2] = f.z;
         v[4 * c + 3] = f.w;
       }
-      f2_tile_store16(v, i16, a.o_tiles + ((size_t)(tok / kF2Cols) * a.nq + hb) * kF2XTile, tok % kF2Cols);
+      f2_store_column(v, i16, a.o_tiles, tok, hb, a.nq, a.o_tile_cols != 0);
     }
   }
 }
@@ -426,7 +426,8 @@ size_t attn_prefill_partial_floats(int nkv, int tokens, int ranges) {
 hipError_t launch_attention_prefill(AttnArgs a, float *partials, int ranges, hipStream_t s) {
   if (a.nkv < 1 || a.nq % a.nkv != 0 || a.nq / a.nkv > kAttnMaxGroup || a.capacity < 1 || a.window < 0 ||
       a.tokens < 1 || a.tokens > kMaxChunkTokens || a.tokens > a.capacity || a.prep || ranges < 1 ||
-      ranges > kAttnPrefillMaxRanges || (!a.q && !a.q_half))
+      ranges > kAttnPrefillMaxRanges || (!a.q && !a.q_half) ||
+      (a.o_tiles && a.o_tile_cols && a.o_tile_cols < a.tokens))
     return hipErrorInvalidValue;
   a.chunks = ranges;
   const size_t slots = (size_t)a.tokens * a.nkv * ranges * kAttnMaxGroup;
@@ -440,7 +441,8 @@ hipError_t launch_attention_prefill(AttnArgs a, float *partials, int ranges, hip
   hipLaunchKernelGGL(attn_prefill_kernel, dim3(per_xcd * kXcds), dim3(256), 0, s, a, blocks, items);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  const int merge_cols = a.o_tiles ? (a.tokens + kF2Cols - 1) / kF2Cols * kF2Cols : a.tokens;
+  const int tile_cols = a.o_tile_cols ? a.o_tile_cols : (a.tokens + kF2Cols - 1) / kF2Cols * kF2Cols;
+  const int merge_cols = a.o_tiles ? tile_cols : a.tokens;
   hipLaunchKernelGGL(attn_merge_slices_kernel, dim3((a.nq + 3) / 4, merge_cols), dim3(256), 0, s, a);
   return hipGetLastError();
 }

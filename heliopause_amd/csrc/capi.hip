@@ -49,7 +49,8 @@ struct Handle {
   uint32_t *f16_flag = nullptr;  // set by the Q6_K repack (launch_repack)
   // The matrix-core kernels' f16 weight operands sc * q are exact for every
   // block (always for Q4_K; for Q6_K unless the repack set f16_flag).  When
-  // false the launches that would use matrix cores run the vector-ALU kernels.
+  // false the single-operand matrix-core kernels leave the launch to the fast
+  // prefill and mid kernels (two exact operands) or the vector ALU.
   bool f16_exact = true;
   uint32_t generation = 0;
   bool live = false;
@@ -320,13 +321,26 @@ constexpr size_t kFastMinCols = 64;
 // Q6_K weight with scales beyond those, Handle::f16_exact).
 struct MfmaFit {
   bool tiles, f16;
+  long long segs;  // the launch's 16-row segments
 };
+
+// The mid kernels (kquant_mid.hip): every column of a launch on the matrix
+// cores, bit-exact.  They take the column counts below the fast kernel's, and
+// every count of the host-pointer calls: from five columns on (measured against
+// the vector-ALU and kquant_mfma kernels: five columns of Q/K/V 14.3 -> 9.5 us,
+// of the FFN 61.8 -> 36.0; at four O 6.9 -> 9.1, Q/K/V 9.8 -> 9.8, with the
+// launch that writes the activation tiles), and from two on for launches of 16
+// segments a CU (the head, two columns 176 -> 155 us, three 223 -> 164; heads
+// of 2000 segments the same either way).
+constexpr size_t kMidMinCols = 5;
+constexpr size_t kMidMinColsLarge = 2;
+constexpr int kMidLargeSegs = 16;  // 16-row segments per CU
 
 // 0: not a prefill launch, 1: bit-exact prefill, 2: fast prefill
 // The automatic fast kernel takes every Q6_K weight (with full-range scales
 // as two exact operands, MfmaLaunch::wide6); the other prefill kernels, and
 // the forced fast one, take launches with single f16 operands only.
-int prefill_kind(size_t cols, MfmaFit fit) {
+int chunk_kind(size_t cols, MfmaFit fit) {
   const State &s = st();
   const int forced = s.matvec_kernel;
   if (!fit.tiles) return 0;
@@ -342,6 +356,18 @@ int prefill_kind(size_t cols, MfmaFit fit) {
   if (cols >= kFastMinCols && fast_fits && !s.host_exact) return 2;
   if (cols >= kPrefillMinCols && exact_fits) return 1;
   return 0;
+}
+
+// The same, or 3: the mid kernel.  A launch whose activation tiles cannot be
+// had (a captured call that no earlier call has sized scratch for, which the
+// kernels of chunk_kind 0 do not need) runs as chunk_kind says: the same bits.
+int prefill_kind(size_t cols, MfmaFit fit) {
+  const State &s = st();
+  const int kind = chunk_kind(cols, fit);
+  const size_t least = fit.segs >= (long long)kMidLargeSegs * s.num_cus ? kMidMinColsLarge : kMidMinCols;
+  if (s.matvec_kernel == 0 && kind != 2 && fit.tiles && cols >= least && cols <= 65535 && mid_lds_bytes() <= s.max_lds)
+    return 3;
+  return kind;
 }
 
 bool use_mfma(size_t cols, int nb, int tiles16, bool f16ok) {
@@ -391,11 +417,12 @@ int g_nb_of(Handle *const *hs) { return hs[0]->g.nb; }
 // matrix-core kernels' 32-bit tile offsets (under 4 GiB).
 MfmaFit mfma_fit(size_t count, Handle *const *hs) {
   bool tiles = false;
-  MfmaFit f{true, true};
+  MfmaFit f{true, true, 0};
   for (size_t i = 0; i < count; i++) tiles = tiles || !hs[i]->segs;
   for (size_t i = 0; i < count; i++) {
-    if (tiles && hs[i]->byte_length >= ((size_t)1 << 32)) f = MfmaFit{false, false};
+    if (tiles && hs[i]->byte_length >= ((size_t)1 << 32)) f.tiles = f.f16 = false;
     if (!hs[i]->f16_exact) f.f16 = false;
+    f.segs += (long long)((hs[i]->row_count + 15) / 16);
   }
   return f;
 }
@@ -455,13 +482,21 @@ bool use_wide_pair(Handle *const *hs, size_t cols) {
 int32_t run_norm(const float *y, int rows, int n, const float *w_post, const float *x_res, float scale, float *x_out,
                  const float *w_next, float *next_out, double eps, hipStream_t stream, uint8_t *q8img = nullptr,
                  uint8_t *xt = nullptr, const PrefillParts *y_parts = nullptr, bool next_image_only = false,
-                 bool x16 = false);
+                 bool x16 = false, int xt_cols = 0);
+
+// Scratch for the mid kernel's activation tiles, or null when there is none.
+uint8_t *mid_scratch(size_t input_size, size_t cols, hipStream_t stream) {
+  void *p = nullptr;
+  const int32_t rc = stream_scratch(stream, kScratchPrefill, mid_bytes((int)input_size, (int)cols), &p);
+  return rc == HP_OK ? static_cast<uint8_t *>(p) : nullptr;
+}
 
 // Whether a one-column launch over these weights runs a vector-ALU kernel,
-// which can form its input with the norm prologue.
-bool norm_prologue_ok(size_t count, Handle *const *hs, size_t cols) {
+// which can form its input with the norm prologue.  kind: the launch's prefill
+// kind.
+bool norm_prologue_ok(size_t count, Handle *const *hs, size_t cols, int kind) {
   const MfmaFit fit = mfma_fit(count, hs);
-  if (cols != 1 || hs[0]->g.nb > 16 || prefill_kind(cols, fit) != 0) return false;
+  if (cols != 1 || hs[0]->g.nb > 16 || kind != 0) return false;
   int tiles16 = 0;
   for (size_t i = 0; i < count; i++) tiles16 += (int)((hs[i]->row_count + 15) / 16);
   return !use_mfma(cols, hs[0]->g.nb, tiles16, fit.f16);
@@ -469,9 +504,9 @@ bool norm_prologue_ok(size_t count, Handle *const *hs, size_t cols) {
 
 // Whether a launch of `cols` columns (2 or more) runs the vector-ALU kernels
 // in one chunk, so it can take its input as a pre-quantised image.
-bool image_input_ok(size_t count, Handle *const *hs, size_t cols) {
+bool image_input_ok(size_t count, Handle *const *hs, size_t cols, int kind) {
   const MfmaFit fit = mfma_fit(count, hs);
-  if (cols < 2 || prefill_kind(cols, fit) != 0) return false;
+  if (cols < 2 || kind != 0) return false;
   int tiles16 = 0;
   for (size_t i = 0; i < count; i++) tiles16 += (int)((hs[i]->row_count + 15) / 16);
   return !use_mfma(cols, hs[0]->g.nb, tiles16, fit.f16) && cols_per_launch(hs[0]->g, st().max_lds) >= (int)cols;
@@ -493,11 +528,16 @@ int32_t run_matvec(size_t count, Handle *const *hs, const float *d_input, size_t
   State &s = st();
   if (cols == 0) return HP_OK;
   if (tail_in && !tail_in->part) tail_in = nullptr;
-  const bool image_ok = s.images && cols >= 2 && image_input_ok(count, hs, cols);
   const MfmaFit fit = mfma_fit(count, hs);
-  const bool wide = prefill_kind(cols, fit) == 0 && use_wide(count, hs, cols);
+  int kind = prefill_kind(cols, fit);
+  uint8_t *pre = nullptr;  // the prefill kernels' scratch
+  if (kind == 3) {
+    pre = mid_scratch(input_size, cols, stream);
+    if (!pre) kind = chunk_kind(cols, fit);
+  }
+  const bool image_ok = s.images && cols >= 2 && image_input_ok(count, hs, cols, kind);
+  const bool wide = kind == 0 && use_wide(count, hs, cols);
   const bool wide_norm = wide && cols == 1 && g_nb_of(hs) <= 16;  // the wide kernel's norm prologue
-  const int kind = prefill_kind(cols, fit);
   if (kind && cols > 65535) return fail(HP_ERR_SHAPE, "too many columns");
   // a deferred GeGLU tail is completed by the fast prefill kernel's pre-pass
   if (tail_in && (kind != 2 || norm || tiles_in)) return fail(HP_ERR_ARG, "deferred GeGLU tail needs the fast prefill");
@@ -516,8 +556,7 @@ int32_t run_matvec(size_t count, Handle *const *hs, const float *d_input, size_t
     l.out[i] = d_outs[i];
   }
   l.wide6 = !fit.f16;
-  uint8_t *pre = nullptr;  // the prefill kernels' scratch
-  if (kind) {
+  if (kind && !pre) {
     const size_t need = kind == 2 ? prefill_fast_bytes(l, s.num_cus) : prefill_q8k_bytes((int)input_size, (int)cols);
     void *p = nullptr;
     int32_t rc = stream_scratch(stream, kScratchPrefill, need, &p);
@@ -526,16 +565,17 @@ int32_t run_matvec(size_t count, Handle *const *hs, const float *d_input, size_t
   }
   // the norm kernel below, or the producer of d_input (tiles_in: the prefill
   // attention's slice merge), wrote the fast prefill's tiles
-  bool tiles_ready = s.prefill_folds && tiles_in && kind == 2 && input_size % kQK == 0;
+  bool tiles_ready = s.prefill_folds && tiles_in && kind >= 2 && input_size % kQK == 0;
   const bool y_split = norm_parts && norm_parts->ks > 1;  // the norm's y as partial sums
-  if (norm && (y_split || (wide ? !wide_norm : !norm_prologue_ok(count, hs, cols)))) {
+  if (norm && (y_split || (wide ? !wide_norm : !norm_prologue_ok(count, hs, cols, kind)))) {
     uint8_t *img = image_ok && img_scratch ? img_scratch : nullptr;
-    tiles_ready = s.prefill_folds && kind == 2 && input_size % kQK == 0;
-    // with its tiles written, the fast prefill kernel does not read the f32
+    tiles_ready = s.prefill_folds && kind >= 2 && input_size % kQK == 0;
+    // with its tiles written, the prefill kernel does not read the f32
     // input (kept for an image: storing it measured faster for the drafts)
     int32_t rc = run_norm(norm->y, (int)cols, (int)input_size, norm->w_post, norm->mode == 2 ? norm->x_res : nullptr,
                           norm->scale, norm->x_out, norm->w_next, norm_scratch, norm->eps, stream, img,
-                          tiles_ready ? pre : nullptr, norm_parts, tiles_ready, true);
+                          tiles_ready ? pre : nullptr, norm_parts, tiles_ready, true,
+                          kind == 3 ? mid_pad_cols((int)cols) : 0);
     if (rc != HP_OK) return rc;
     d_input = norm_scratch;
     norm = nullptr;
@@ -570,7 +610,10 @@ int32_t run_matvec(size_t count, Handle *const *hs, const float *d_input, size_t
   a.total_units = a.Rh ? (rows_all + a.Rh - 1) / a.Rh : 0;
   if (kind) {
     hipEvent_t e1 = prof_begin(stream);
-    if (kind == 2) {
+    if (kind == 3) {
+      if (!tiles_ready) HP_HIP_TRY(launch_mid_tiles(d_input, (int)input_size, (int)cols, mid_pad_cols((int)cols), pre, stream));
+      HP_HIP_TRY(launch_mid(l, pre, nullptr, nullptr, s.num_cus, stream));
+    } else if (kind == 2) {
       const size_t part_bytes = defer ? prefill_fast_part_bytes(l, s.num_cus) : 0;
       if (part_bytes) {
         void *p = nullptr;
@@ -586,7 +629,7 @@ int32_t run_matvec(size_t count, Handle *const *hs, const float *d_input, size_t
       HP_HIP_TRY(launch_prefill(l, pre, s.num_cus, stream));
     }
     prof_end(HP_KERNEL_MATVEC, e1, stream);
-    s.launches += kind == 2 ? prefill_fast_launches(l, s.num_cus) - (tiles_ready ? 1 : 0) : 2;
+    s.launches += (kind == 2 ? prefill_fast_launches(l, s.num_cus) : 2) - (tiles_ready ? 1 : 0);
     s.matmul_calls++;
     return HP_OK;
   }
@@ -679,14 +722,20 @@ int32_t run_matvec_geglu(Handle *hg, Handle *hu, const float *d_input, size_t in
   const int tiles16 = 2 * (int)((rows + 15) / 16);
   Handle *pair[2] = {hg, hu};
   const MfmaFit fit = mfma_fit(2, pair);
-  const bool wide = prefill_kind(cols, fit) == 0 && hg->type == hu->type && use_wide_pair(pair, cols);
-  const bool fused = !wide && cols <= 4 && s.matvec_kernel <= 1 && !use_mfma(cols, g.nb, tiles16, fit.f16) &&
+  int kind = prefill_kind(cols, fit);
+  uint8_t *pre = nullptr;  // the prefill kernels' scratch, tiles first
+  if (kind == 3) {
+    pre = mid_scratch(input_size, cols, stream);
+    if (!pre) kind = chunk_kind(cols, fit);
+  }
+  const bool mid = kind == 3;  // gate and up segments in one workgroup, GeGLU in its last sums
+  const bool wide = kind == 0 && hg->type == hu->type && use_wide_pair(pair, cols);
+  const bool fused = !wide && !mid && cols <= 4 && s.matvec_kernel <= 1 && !use_mfma(cols, g.nb, tiles16, fit.f16) &&
                      !use_half((int)cols, g, 2 * hg->tiles, (int)(2 * rows)) && cols_per_launch(g, s.max_lds) >= (int)cols;
   // fast prefill: gate and up rows in one tile, GeGLU in its epilogue
-  const bool fast = prefill_kind(cols, fit) == 2 && hg->type == hu->type;
+  const bool fast = kind == 2 && hg->type == hu->type;
   MfmaLaunch l{};
-  uint8_t *pre = nullptr;  // its scratch, tiles first
-  if (fast) {
+  if (fast || mid) {
     l.count = 2;
     l.k = (int)input_size;
     l.S = g.S;
@@ -700,21 +749,33 @@ int32_t run_matvec_geglu(Handle *hg, Handle *hu, const float *d_input, size_t in
       l.rows[i] = (int)rows;
     }
     l.wide6 = !fit.f16;
+  }
+  if (fast) {
     void *p = nullptr;
     int32_t rc = stream_scratch(stream, kScratchPrefill, prefill_fast_geglu_bytes(l, s.num_cus), &p);
     if (rc != HP_OK) return rc;
     pre = static_cast<uint8_t *>(p);
   }
-  bool tiles_ready = false;  // the norm kernel wrote the fast prefill's tiles
+  bool tiles_ready = false;  // the norm kernel wrote the launch's tiles
   const bool y_split = norm_parts && norm_parts->ks > 1;  // the norm's y as partial sums
   if (norm && (y_split || !((fused || wide) && cols == 1 && g.nb <= 16))) {
-    tiles_ready = s.prefill_folds && fast && input_size % kQK == 0;
+    tiles_ready = s.prefill_folds && (fast || mid) && input_size % kQK == 0;
     int32_t rc = run_norm(norm->y, (int)cols, (int)input_size, norm->w_post, norm->mode == 2 ? norm->x_res : nullptr,
                           norm->scale, norm->x_out, norm->w_next, norm_scratch, norm->eps, stream, nullptr,
-                          tiles_ready ? pre : nullptr, norm_parts, tiles_ready, true);
+                          tiles_ready ? pre : nullptr, norm_parts, tiles_ready, true,
+                          mid ? mid_pad_cols((int)cols) : 0);
     if (rc != HP_OK) return rc;
     d_input = norm_scratch;
     norm = nullptr;
+  }
+  if (mid) {
+    hipEvent_t e1 = prof_begin(stream);
+    if (!tiles_ready) HP_HIP_TRY(launch_mid_tiles(d_input, (int)input_size, (int)cols, mid_pad_cols((int)cols), pre, stream));
+    HP_HIP_TRY(launch_mid(l, pre, s.gelu_lut, d_out, s.num_cus, stream));
+    prof_end(HP_KERNEL_MATVEC, e1, stream);
+    s.launches += tiles_ready ? 1 : 2;
+    s.matmul_calls++;
+    return HP_OK;
   }
   if (wide) {
     MatvecArgs a{};
@@ -1131,8 +1192,9 @@ int32_t run_attention(AttnArgs a, float *partials, hipStream_t stream) {
 
 int32_t run_norm(const float *y, int rows, int n, const float *w_post, const float *x_res, float scale, float *x_out,
                  const float *w_next, float *next_out, double eps, hipStream_t stream, uint8_t *q8img,
-                 uint8_t *xt, const PrefillParts *y_parts, bool next_image_only, bool x16) {
+                 uint8_t *xt, const PrefillParts *y_parts, bool next_image_only, bool x16, int xt_cols) {
   NormArgs a{};
+  a.xt_cols = xt_cols;
   a.x16 = x16 ? 1 : 0;
   a.q8img = q8img;
   a.xt = xt;
@@ -2566,11 +2628,17 @@ int32_t hp_hip_decode_layers_device(const hp_hip_decode_layer_t *layers, size_t 
       } else {
         const int ranges = attn_prefill_ranges((int)Mc, L.attention.head_count, L.attention.head_count_kv,
                                                L.attention.capacity, s.num_cus);
-        // O on the fast prefill kernel: the slice merge writes its
+        // O on the fast prefill or the mid kernel: the slice merge writes its
         // activation tiles into O's prefill scratch (the pre-pass launch
         // they replace would write the same bytes there)
-        if (s.prefill_folds && prefill_kind(Mc, mfma_fit(1, &H.o)) == 2 && H.o->input_size % kQK == 0 &&
-            H.o->input_size == (size_t)L.attention.head_count * kHeadDim) {
+        const int o_kind = prefill_kind(Mc, mfma_fit(1, &H.o));
+        const bool o_fold = s.prefill_folds && o_kind >= 2 && H.o->input_size % kQK == 0 &&
+                            H.o->input_size == (size_t)L.attention.head_count * kHeadDim;
+        if (o_fold && o_kind == 3) {
+          aa.o_tiles = mid_scratch(H.o->input_size, Mc, strm);
+          aa.o_tile_cols = mid_pad_cols((int)Mc);
+          o_tiles = aa.o_tiles != nullptr;
+        } else if (o_fold) {
           MfmaLaunch lo{};
           lo.count = 1;
           lo.k = (int)H.o->input_size;

@@ -85,7 +85,7 @@ __global__ __launch_bounds__(256) void norm_residual_kernel(const NormArgs a) {
 #pragma unroll
     for (int e = 0; e < 16; e++) z[e] = 0.0f;
     for (int b = g; b < nb; b += 16)
-      f2_tile_store16(z, i16, a.xt + ((size_t)(blockIdx.x / kF2Cols) * nb + b) * kF2XTile, blockIdx.x % kF2Cols);
+      f2_store_column(z, i16, a.xt, blockIdx.x, b, nb, a.xt_cols != 0);
     return;
   }
   const size_t row = (size_t)blockIdx.x * a.n;
@@ -169,8 +169,7 @@ __global__ __launch_bounds__(256) void norm_residual_kernel(const NormArgs a) {
                       reinterpret_cast<float *>(a.q8img + (size_t)a.rows * nb * kQ8BlockBytes) + q);
         }
         if (a.xt)
-          f2_tile_store16(xv, i16, a.xt + ((size_t)(blockIdx.x / kF2Cols) * nb + b) * kF2XTile,
-                          blockIdx.x % kF2Cols);
+          f2_store_column(xv, i16, a.xt, blockIdx.x, b, nb, a.xt_cols != 0);
       }
     }
   }
@@ -195,7 +194,7 @@ __global__ __launch_bounds__(256) void norm_residual_x16_kernel(const NormArgs a
 #pragma unroll
     for (int e = 0; e < 16; e++) z[e] = 0.0f;
     if (g < nb)
-      f2_tile_store16(z, i16, a.xt + ((size_t)(blockIdx.x / kF2Cols) * nb + g) * kF2XTile, blockIdx.x % kF2Cols);
+      f2_store_column(z, i16, a.xt, blockIdx.x, g, nb, a.xt_cols != 0);
     return;
   }
   const bool live = g < nb;
@@ -247,7 +246,7 @@ __global__ __launch_bounds__(256) void norm_residual_x16_kernel(const NormArgs a
                 reinterpret_cast<float *>(a.q8img + (size_t)a.rows * nb * kQ8BlockBytes) + q);
   }
   if (a.xt)
-    f2_tile_store16(o, i16, a.xt + ((size_t)(blockIdx.x / kF2Cols) * nb + g) * kF2XTile, blockIdx.x % kF2Cols);
+    f2_store_column(o, i16, a.xt, blockIdx.x, g, nb, a.xt_cols != 0);
 }
 
 // One wave per head: query heads (norm with wq, RoPE, f32 out or its f16
@@ -772,7 +771,8 @@ hipError_t launch_norm_residual(const NormArgs &a, hipStream_t s) {
   if ((a.q8img || a.xt) && (a.n % kQK != 0 || !a.next_out)) return hipErrorInvalidValue;
   if (a.next_image_only && !a.q8img && !a.xt) return hipErrorInvalidValue;
   if (a.y_ks > kNormParts || (a.y_ks > 1 && a.y_stride < (size_t)a.rows * a.n)) return hipErrorInvalidValue;
-  const int grid = a.xt ? (a.rows + kF2Cols - 1) / kF2Cols * kF2Cols : a.rows;
+  if (a.xt && a.xt_cols && a.xt_cols < a.rows) return hipErrorInvalidValue;
+  const int grid = !a.xt ? a.rows : a.xt_cols ? a.xt_cols : (a.rows + kF2Cols - 1) / kF2Cols * kF2Cols;
   if (a.x16 && a.next_out && a.n % kQK == 0 && a.n <= 16 * kQK) {
     // rows that feed a projection: the block-per-group form
     hipLaunchKernelGGL(norm_residual_x16_kernel, dim3(grid), dim3(256), 0, s, a);

@@ -485,6 +485,18 @@ hipError_t launch_prefill_fast(const MfmaLaunch &l, const float *x, uint8_t *scr
                                bool tiles_ready = false, PrefillParts *defer = nullptr,
                                const GegluTail *tail = nullptr);
 
+// Mid kernel (kquant_mid.hip; bit-exact, any column count up to 65535, made
+// for 2 to 63): reads the mid_bytes(k, cols) of 16-column activation tiles
+// (hp_f2tile.h) of mid_pad_cols(cols) columns, written by launch_mid_tiles,
+// the norm kernel (NormArgs::xt) or the attention's slice merge.  With pair_out (two
+// weights of equal rows, gate and up): pair_out[m][r] = fround(gelu(gate) * up).
+size_t mid_bytes(int k, int cols);
+size_t mid_lds_bytes();
+int mid_pad_cols(int cols);
+hipError_t launch_mid_tiles(const float *x, int k, int cols, int pad_cols, uint8_t *xt, hipStream_t s);
+hipError_t launch_mid(const MfmaLaunch &l, const uint8_t *xt, const uint16_t *gelu_lut, float *pair_out, int num_cus,
+                      hipStream_t s);
+
 // The gelu table (65536 f16 entries, hp_gelu.h gelu_lut) for the constant c.
 hipError_t launch_gelu_lut(double c, uint16_t *lut, hipStream_t s);
 // GeGLU of cols columns of `rows` (a multiple of 256) that also writes the
@@ -515,6 +527,7 @@ struct NormArgs {
   // (hp_f2tile.h; row r is column r; the grid covers whole 64-column tiles,
   // workgroups past `rows` write their padding columns as zeros)
   uint8_t *xt;
+  int xt_cols;  // not 0: the mid kernel's 16-column tiles, of this many columns (at least rows)
   // x16: 16-lane groups hold whole 256-element blocks (norm_residual_x16_kernel;
   // n a multiple of 256, at most 4096): the norms that feed a projection
   int x16;
@@ -567,6 +580,7 @@ struct AttnArgs {
   // whole 64-column tiles, padding columns as zeros), the next projection's
   // input
   uint8_t *o_tiles;
+  int o_tile_cols;  // not 0: the mid kernel's 16-column tiles, of this many columns (at least tokens)
   const float *wq, *wk, *freq_factors;
   _Float16 *k_cache, *v_cache;
   const int *position;
