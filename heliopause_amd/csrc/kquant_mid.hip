@@ -62,43 +62,78 @@ __device__ __forceinline__ const uint8_t *group_tiles(const uint8_t *xt, int cg,
 // ---- class pairs: launches with few segments --------------------------------
 //
 // A workgroup of four waves takes one segment and one column group; wave w
-// keeps classes 2w and 2w + 1 (640 waves for the 2560 rows of O or down, where
-// a wave per segment would leave most SIMDs empty) and a quarter of the min
-// chain's columns.  The waves' classes are disjoint, so neither weights nor
+// keeps classes 2w and 2w + 1 (KL = 2; 640 waves for the 2560 rows of O or
+// down, where a wave per segment would leave most SIMDs empty) and a quarter of
+// the min chain's columns.  With no more workgroups than CUs, one wave a SIMD
+// waits on each of its own instructions, and eight waves of one class (KL = 1)
+// are faster over long rows although they unpack every header twice as often.  The waves' classes are disjoint, so neither weights nor
 // activations have a second reader in the workgroup: both go straight from
 // global memory to registers, mid_depth blocks ahead, with no stage in LDS and
 // no barrier until the chains meet (measured against activations copied
 // through a ring of LDS stages by waves of their own: the copies, 46 bytes per
-// clock and CU, bounded it).  Per block and wave the loads cost the L1 64 to
-// 128 bytes a clock times the column sets, so what a row shares is loaded
-// once and spread by lane swaps: its header as one dword per lane, a column's
-// d as one dword per lane of a four-lane group.
+// clock and CU, bounded it).  Those loads share the CU's L1 (64 bytes and one
+// address group a clock), so what lanes share is loaded once and spread by
+// lane swaps: a row's header as one dword per lane, a column's d as one dword
+// per lane of a four-lane group.
 constexpr int mid_depth(int C) { return C == 1 ? 5 : 4; }
 
 // The chains' exchange at the end: [9][16 C columns][16 rows, padded to 20]
 // floats per segment (the padding spreads a wave's store over all banks).
 constexpr int kMidRowPad = 20;
 
-// One block of a lane's operands: row n = lane % 16 of the segment, quarter
-// q = lane / 16 (elements j = 2q, 2q + 1) of classes 2w and 2w + 1; the
-// activations of column nrot(n) of each set.
-template <int C, bool Q4>
-struct MidRaw;
-template <int C>
-struct MidRaw<C, true> {
-  uint32_t hdr;    // dword q of the row's header (d | dmin, 12 scale/min bytes)
-  uint32_t ql[2];  // quant dwords D[q][2w + g]
-  uint4 B[2][C], bm[C];
-  float dx[C];
+// One block of a lane's weights: row n = lane % 16 of the segment, quarter
+// q = lane / 16 (elements j = 2q, 2q + 1) of classes l = KL w + g, g < KL.
+template <int KL, bool Q4>
+struct MidW;
+template <int KL>
+struct MidW<KL, true> {
+  uint32_t hdr;     // dword q of the row's header (d | dmin, 12 scale/min bytes)
+  uint32_t ql[KL];  // quant dwords D[q][l]
 };
-template <int C>
-struct MidRaw<C, false> {
+template <int KL>
+struct MidW<KL, false> {
   uint32_t gs, d16;  // scales of groups 4q .. 4q + 3, f16 d
-  uint32_t ql[2];    // low bits D[q][2w + g]
-  uint2 qh;          // high bits Dqh[q / 2][2w], Dqh[q / 2][2w + 1] (tiles: ^ 0xAA per byte)
-  uint4 B[2][C];
+  uint32_t ql[KL];   // low bits D[q][l]
+  uint32_t qh[KL];   // high bits Dqh[q / 2][l] (tiles: ^ 0xAA per byte)
+};
+// The block as loaded.  A segment stores a row's four dwords of a class side
+// by side; loaded where its fragment needs it, lane (n, q) dword 4 n + q, a
+// dword load touches four times the bytes it takes (16-byte strides: the L1's
+// address unit was busy 84 % of the down launch).  So lane i loads dword i
+// (wq: quant dwords of class l, wh: high-bit dwords, ws: header or
+// scales) and mid_place spreads them.  From tiles: already in place, w.
+template <int C, int KL, bool Q4, bool TILE>
+struct MidRaw {
+  MidW<KL, Q4> w;
+  uint32_t wq[KL], wh, ws, d16;
+  uint4 B[KL][C], bm[C];  // activations of column nrot(n) of each set
   float dx[C];
 };
+
+// Lane 16 q + n's weights (classes l0 ..) from the lanes that loaded them.
+template <int C, int KL, bool Q4, bool TILE>
+__device__ __forceinline__ MidW<KL, Q4> mid_place(const MidRaw<C, KL, Q4, TILE> &r, uint32_t n, uint32_t q,
+                                                  uint32_t l0) {
+  if constexpr (TILE) {
+    return r.w;
+  } else {
+    auto from = [](uint32_t lane, uint32_t v) {
+      return (uint32_t)__builtin_amdgcn_ds_bpermute((int)(4u * lane), (int)v);
+    };
+    MidW<KL, Q4> w;
+#pragma unroll
+    for (int g = 0; g < KL; g++) w.ql[g] = from(4u * n + q, r.wq[g]);
+    if constexpr (Q4) {
+      w.hdr = from(4u * n + q, r.ws);
+    } else {
+#pragma unroll
+      for (int g = 0; g < KL; g++) w.qh[g] = from(4u * n + 2u * (q >> 1) + ((l0 + g) & 1u), r.wh);
+      w.gs = from(4u * n + q, r.ws);
+      w.d16 = r.d16;
+    }
+    return w;
+  }
+}
 
 template <class T>
 __device__ __forceinline__ T ldg(const uint8_t *base, uint32_t off) {
@@ -135,68 +170,73 @@ __device__ __forceinline__ float quad_lane(float v) {
 // the Q4_K min chain of a quarter of the columns.  Sum j of lane (n, q) is row
 // n, column 16 cs + 4q + (j + w) % 4: the columns are turned by w within each
 // four, so that sum 0, the min chain's, is another column in each wave.
-template <int C, bool Q4, bool TILE>
-__device__ __forceinline__ void mid_tile(float (&s)[2][C][4], float (&f)[C], const MidWeight &W, int tt, int nb,
+template <int C, int KL, bool Q4, bool TILE>
+__device__ __forceinline__ void mid_tile(float (&s)[KL][C][4], float (&f)[C], const MidWeight &W, int tt, int nb,
                                          int S, int R, const uint8_t *xt, int w, int lane) {
   constexpr int PD = mid_depth(C), segb = Q4 ? 2304 : 3360;
+  const uint32_t l0 = KL * w;
   const uint32_t n = lane & 15, q = lane >> 4;
   const uint32_t exp = magic_nib_exp();
   const QuarterMasks mq = quarter_masks(q);
   TileRow tr{};
   if constexpr (TILE) tr = tile_row(min(16 * tt + (int)n, W.rows - 1), W.rows, nb, S, R, Q4 ? 9 : 13);
   // lane offsets: within a segment, and within an activation tile
-  const uint32_t unit = 16u * (n + 16u * w), oq = (Q4 ? 256u : 288u) + unit + 4u * q;
-  const uint32_t oh = Q4 ? 16u * n + 4u * q : 2336u + unit + 8u * (q >> 1);
-  const uint32_t os = 16u * n + 4u * q, od = 256u + 2u * n;
+  const uint32_t os = 4u * (uint32_t)lane, oh = 2336u + 256u * (l0 >> 1) + os;
+  const uint32_t oq = (Q4 ? 256u : 288u) + 1024u * (l0 & 1u) + 256u * (l0 >> 1) + os;  // (class l0 + 1 is 1024 on)
+  const uint32_t od = 256u + 2u * n;
   const uint32_t nrot = (n & ~3u) | ((n + w) & 3u);
-  const uint32_t ox = ((8u * w + q) * 16u + nrot) * 16u;        // class 2w; class 2w + 1 is 1024 on
+  const uint32_t ox = ((4u * l0 + q) * 16u + nrot) * 16u;       // class l0; class l0 + 1 is 1024 on
   const uint32_t ob = 8192u + ((q & 1u) * 16u + nrot) * 16u;    // (quarters 2, 3 meet zero mins)
   const uint32_t ods = 8704u + 4u * (4u * q + ((n + w) & 3u));
   auto load = [&](int b) {  // unconditional: a block past the last re-reads it
     b = min(b, nb - 1);
-    MidRaw<C, Q4> r;
+    MidRaw<C, KL, Q4, TILE> r;
     if constexpr (TILE) {
-      // D[q][2w], D[q][2w + 1] are the 8-byte pair at byte 8 (w % 2) of quant chunk 2q + w / 2
+      // D[q][l] is dword l % 4 of quant chunk 2q + l / 4
       int i, sl;
       block_split(b, S, i, sl);
-      const uint32_t off = tr.base + (uint32_t)i * tr.iter + 16u * (uint32_t)sl, half = 8u * (w & 1u), c = w >> 1;
-      const uint2 p = ldg<uint2>(W.wt, off + ((Q4 ? 1u : 0u) + 2u * q + c) * tr.chunk + half);
-      r.ql[0] = p.x;
-      r.ql[1] = p.y;
+      const uint32_t off = tr.base + (uint32_t)i * tr.iter + 16u * (uint32_t)sl, at = 4u * (l0 & 3u), c = l0 >> 2;
+      const uint32_t lq = off + ((Q4 ? 1u : 0u) + 2u * q + c) * tr.chunk + at;
+      const uint32_t lh = off + (8u + 2u * (q >> 1) + c) * tr.chunk + at;
+#pragma unroll
+      for (int g = 0; g < KL; g++) r.w.ql[g] = ldg<uint32_t>(W.wt, lq + 4u * g);
       if constexpr (Q4) {
-        r.hdr = ldg<uint32_t>(W.wt, off + 4u * q);
+        r.w.hdr = ldg<uint32_t>(W.wt, off + 4u * q);
       } else {
-        r.gs = ldg<uint32_t>(W.wt, off + 12u * tr.chunk + 4u * q);
-        r.d16 = W.dplane[tr.dbase + (uint32_t)i * tr.diter + (uint32_t)sl];
-        r.qh = ldg<uint2>(W.wt, off + (8u + 2u * (q >> 1) + c) * tr.chunk + half);
+        r.w.gs = ldg<uint32_t>(W.wt, off + 12u * tr.chunk + 4u * q);
+        r.w.d16 = W.dplane[tr.dbase + (uint32_t)i * tr.diter + (uint32_t)sl];
+#pragma unroll
+        for (int g = 0; g < KL; g++) r.w.qh[g] = ldg<uint32_t>(W.wt, lh + 4u * g);
       }
     } else {
       const uint8_t *seg = W.seg + ((size_t)b * W.tiles + tt) * segb;
-      r.ql[0] = ldg<uint32_t>(seg, oq);
-      r.ql[1] = ldg<uint32_t>(seg + 1024, oq);
-      if constexpr (Q4) {
-        r.hdr = ldg<uint32_t>(seg, oh);
-      } else {
-        r.qh = ldg<uint2>(seg, oh);
-        r.gs = ldg<uint32_t>(seg, os);
+#pragma unroll
+      for (int g = 0; g < KL; g++) r.wq[g] = ldg<uint32_t>(seg + 1024 * g, oq);
+      r.ws = ldg<uint32_t>(seg, os);
+      if constexpr (!Q4) {
+        r.wh = ldg<uint32_t>(seg, oh);
         r.d16 = ldg<uint16_t>(seg, od);
       }
     }
 #pragma unroll
     for (int cs = 0; cs < C; cs++) {
       const uint8_t *x = xt + ((size_t)cs * nb + b) * kMidXTile;
-      r.B[0][cs] = ldg<uint4>(x, ox);
-      r.B[1][cs] = ldg<uint4>(x + 1024, ox);
+#pragma unroll
+      for (int g = 0; g < KL; g++) r.B[g][cs] = ldg<uint4>(x + 1024 * g, ox);
       if constexpr (Q4) r.bm[cs] = ldg<uint4>(x, ob);
       r.dx[cs] = ldg<float>(x, ods);
     }
     return r;
   };
-  auto compute = [&](const MidRaw<C, Q4> &r) {
-    half8 a[2], odd[2], mins;
+  // block b's products from its weights v and activations r; block b + 1's
+  // weights (rn) are put in place meanwhile
+  MidW<KL, Q4> v;
+  auto compute = [&](const MidRaw<C, KL, Q4, TILE> &r, const MidRaw<C, KL, Q4, TILE> &rn) {
+    const MidW<KL, Q4> vn = mid_place(rn, n, q, l0);
+    half8 a[KL], odd[KL], mins;
     float dw, dmw = 0.0f;
     if constexpr (Q4) {
-      const uint4 hdr = row_gather(r.hdr);
+      const uint4 hdr = row_gather(v.hdr);
       const uint32_t sclo = hdr.y & 0x3F3F3F3Fu;
       const uint32_t schi = (hdr.w & 0x0F0F0F0Fu) | ((hdr.y >> 2) & 0x30303030u);
       const uint32_t sc = ((sclo & mq.lo) | (schi & ~mq.lo)) >> (16 * (q & 1));
@@ -204,8 +244,8 @@ __device__ __forceinline__ void mid_tile(float (&s)[2][C][4], float (&f)[C], con
       const half2v m1024 = (half2v){(_Float16)-1024.0f, (_Float16)-1024.0f};
       const half2v N0 = S0 * m1024, N1 = S1 * m1024;
 #pragma unroll
-      for (int g = 0; g < 2; g++) {
-        const uint32_t d0 = r.ql[g], d8 = d0 >> 8;
+      for (int g = 0; g < KL; g++) {
+        const uint32_t d0 = v.ql[g], d8 = d0 >> 8;
         a[g] = cat(fma2(magic_nib<kNibLo>(d0, exp), S0, N0), fma2(magic_nib<kNibLo>(d8, exp), S0, N0),
                    fma2(magic_nib<kNibHi>(d0, exp), S1, N1), fma2(magic_nib<kNibHi>(d8, exp), S1, N1));
       }
@@ -219,30 +259,30 @@ __device__ __forceinline__ void mid_tile(float (&s)[2][C][4], float (&f)[C], con
     } else {
       half2v S[2];
       uint32_t M[2];
-      q6_split_scales(S, M, r.gs);
+      q6_split_scales(S, M, v.gs);
       const int jj = 2 * (q & 1);
 #pragma unroll
-      for (int g = 0; g < 2; g++) {
-        const uint32_t ql = r.ql[g], qh = (g ? r.qh.y : r.qh.x) ^ (TILE ? 0xAAAAAAAAu : 0u);
+      for (int g = 0; g < KL; g++) {
+        const uint32_t ql = v.ql[g], qh = v.qh[g] ^ (TILE ? 0xAAAAAAAAu : 0u);
         const uint32_t lo = (ql & 0x0F0F0F0Fu) | (((qh >> (2 * jj)) & 0x03030303u) << 4);
         const uint32_t hi = ((ql >> 4) & 0x0F0F0F0Fu) | (((qh >> (2 * jj + 2)) & 0x03030303u) << 4);
         q6_split(a[g], odd[g], lo, hi, S, M);
       }
-      dw = h2f_bits(r.d16);
+      dw = h2f_bits(v.d16);
     }
-    f32x4 D[2][C], sm[C];
+    f32x4 D[KL][C], sm[C];
     const f32x4 zero = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int cs = 0; cs < C; cs++) {
 #pragma unroll
-      for (int g = 0; g < 2; g++) D[g][cs] = mfma(__builtin_bit_cast(half8, r.B[g][cs]), a[g], zero);
+      for (int g = 0; g < KL; g++) D[g][cs] = mfma(__builtin_bit_cast(half8, r.B[g][cs]), a[g], zero);
       if constexpr (Q4) sm[cs] = mfma(__builtin_bit_cast(half8, r.bm[cs]), mins, zero);
     }
     if constexpr (!Q4) {
 #pragma unroll
       for (int cs = 0; cs < C; cs++)
 #pragma unroll
-        for (int g = 0; g < 2; g++) D[g][cs] = mfma(__builtin_bit_cast(half8, r.B[g][cs]), odd[g], D[g][cs]);
+        for (int g = 0; g < KL; g++) D[g][cs] = mfma(__builtin_bit_cast(half8, r.B[g][cs]), odd[g], D[g][cs]);
     }
 #pragma unroll
     for (int cs = 0; cs < C; cs++) {
@@ -252,12 +292,13 @@ __device__ __forceinline__ void mid_tile(float (&s)[2][C][4], float (&f)[C], con
       for (int j = 0; j < 4; j++) {
         const float dd = __fmul_rn(dw, dx[j]);
 #pragma unroll
-        for (int g = 0; g < 2; g++) s[g][cs][j] = __fadd_rn(s[g][cs][j], __fmul_rn(dd, D[g][cs][j]));
+        for (int g = 0; g < KL; g++) s[g][cs][j] = __fadd_rn(s[g][cs][j], __fmul_rn(dd, D[g][cs][j]));
       }
       if constexpr (Q4) f[cs] = __fsub_rn(f[cs], __fmul_rn(__fmul_rn(dmw, dx[0]), sm[cs][0]));
     }
+    v = vn;
   };
-  MidRaw<C, Q4> r[PD];
+  MidRaw<C, KL, Q4, TILE> r[PD];
   // the scheduling barriers keep the loads in block order: the first wait in
   // the loop would otherwise be for all of them
 #pragma unroll
@@ -265,13 +306,14 @@ __device__ __forceinline__ void mid_tile(float (&s)[2][C][4], float (&f)[C], con
     r[i] = load(i);
     __builtin_amdgcn_sched_barrier(0);
   }
+  v = mid_place(r[0], n, q, l0);
   // (blocks past the last are skipped by a branch around them: an exit inside
   // the loop would join its back edge, and the waits at its head would then be
   // for every load)
   for (int b0 = 0; b0 < nb; b0 += PD) {
 #pragma unroll
     for (int i = 0; i < PD; i++) {
-      if (b0 + i < nb) compute(r[i]);
+      if (b0 + i < nb) compute(r[i], r[(i + 1) % PD]);
       r[i] = load(b0 + i + PD);
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -282,15 +324,16 @@ __device__ __forceinline__ void mid_tile(float (&s)[2][C][4], float (&f)[C], con
 // totals meet in the final sum, which stores fround(gelu(gate) * up).
 // TILE: every weight is read from its tiles (a launch with a weight kept in
 // one layout); else from its segments.
-template <int C, bool PAIR, bool TILE>
-__global__ __launch_bounds__(PAIR ? 512 : 256) __attribute__((amdgpu_waves_per_eu(C == 1 ? 3 : 2))) void
+template <int C, int KL, bool PAIR, bool TILE>
+__global__ __launch_bounds__(512 / KL * (PAIR ? 2 : 1)) __attribute__((amdgpu_waves_per_eu(C == 1 ? 3 : 2))) void
 kquant_mid_kernel(const MidArgs a) {
   kernarg_warm<MidArgs>();
   constexpr int cols = 16 * C, kChain = cols * kMidRowPad;
   __shared__ float fin[(PAIR ? 2 : 1) * 9 * kChain];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int grp = PAIR ? wave >> 2 : 0, w = wave & 3;
+  constexpr int kThreads = 512 / KL;  // of a segment
+  const int grp = PAIR ? wave / (8 / KL) : 0, w = wave & (8 / KL - 1);
   // the column groups of a segment are 8 workgroups apart: one XCD, whose L2
   // holds the segment's weights for all of them
   const int G = a.col_groups, tg = blockIdx.x / (8 * G), rem = blockIdx.x - tg * 8 * G;
@@ -305,18 +348,20 @@ kquant_mid_kernel(const MidArgs a) {
     if (a.count > 3 && t >= a.w[3].tile_begin) W = a.w[3];
   }
   const int tt = PAIR ? t : t - W.tile_begin;
-  float s[2][C][4], f[C];
+  float s[KL][C][4], f[C];
 #pragma unroll
   for (int cs = 0; cs < C; cs++) {
     f[cs] = 0.0f;
 #pragma unroll
-    for (int j = 0; j < 4; j++) s[0][cs][j] = s[1][cs][j] = 0.0f;
+    for (int g = 0; g < KL; g++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) s[g][cs][j] = 0.0f;
   }
   const uint8_t *xt = group_tiles<C>(a.xt, cg, a.nb);
   if (W.type == kTypeQ4K)
-    mid_tile<C, true, TILE>(s, f, W, tt, a.nb, a.S, a.R, xt, w, lane);
+    mid_tile<C, KL, true, TILE>(s, f, W, tt, a.nb, a.S, a.R, xt, w, lane);
   else
-    mid_tile<C, false, TILE>(s, f, W, tt, a.nb, a.S, a.R, xt, w, lane);
+    mid_tile<C, KL, false, TILE>(s, f, W, tt, a.nb, a.S, a.R, xt, w, lane);
   {
     const int n = lane & 15, q = lane >> 4;
     float *fg = fin + grp * 9 * kChain + n;
@@ -326,8 +371,8 @@ kquant_mid_kernel(const MidArgs a) {
       for (int j = 0; j < 4; j++) {
         const int col = 16 * cs + 4 * q + ((j + w) & 3);
 #pragma unroll
-        for (int g = 0; g < 2; g++) fg[(2 * w + g) * kChain + col * kMidRowPad] = s[g][cs][j];
-        if (j == 0) fg[8 * kChain + col * kMidRowPad] = f[cs];
+        for (int g = 0; g < KL; g++) fg[(KL * w + g) * kChain + col * kMidRowPad] = s[g][cs][j];
+        if (j == 0 && w < 4) fg[8 * kChain + col * kMidRowPad] = f[cs];
       }
     }
   }
@@ -344,27 +389,26 @@ kquant_mid_kernel(const MidArgs a) {
   if constexpr (PAIR) {
     const bool q4g = a.w[0].type == kTypeQ4K, q4u = a.w[1].type == kTypeQ4K;
     const int rows = a.w[0].rows;
-    for (int col = tid >> 4; col < cols; col += 32) {
+    for (int col = tid >> 4; col < cols; col += kThreads / 8) {
       const int m = cols * cg + col;
       if (row < rows && m < a.cols)
         a.pair_out[(size_t)m * rows + row] = geglu_lut(total(0, q4g, row16, col), total(1, q4u, row16, col), a.gelu_lut);
     }
   } else {
-#pragma unroll
-    for (int cs = 0; cs < C; cs++) {
-      const int col = 16 * cs + (tid >> 4), m = cols * cg + col;
+    for (int col = tid >> 4; col < cols; col += kThreads / 16) {
+      const int m = cols * cg + col;
       const float v = total(0, W.type == kTypeQ4K, row16, col);
       if (row < W.rows && m < a.cols) W.out[(size_t)m * W.rows + row] = v;
     }
   }
 }
 
-template <int C, bool PAIR>
+template <int C, int KL, bool PAIR>
 void launch_mid_kernel(MidArgs a, bool tiles, hipStream_t s) {
   a.col_groups = (a.cols + 16 * C - 1) / (16 * C);
   if (PAIR) a.total_tiles = a.w[0].tiles;
-  auto *k = tiles ? kquant_mid_kernel<C, PAIR, true> : kquant_mid_kernel<C, PAIR, false>;
-  hipLaunchKernelGGL(k, dim3((a.total_tiles + 7) / 8 * 8 * a.col_groups), dim3(PAIR ? 512 : 256), 0, s, a);
+  auto *k = tiles ? kquant_mid_kernel<C, KL, PAIR, true> : kquant_mid_kernel<C, KL, PAIR, false>;
+  hipLaunchKernelGGL(k, dim3((a.total_tiles + 7) / 8 * 8 * a.col_groups), dim3(512 / KL * (PAIR ? 2 : 1)), 0, s, a);
 }
 
 // ---- row waves: launches with many segments ---------------------------------
@@ -781,17 +825,28 @@ hipError_t launch_mid(const MfmaLaunch &l, const uint8_t *xt, const uint16_t *ge
       launch_rows_kernel<2, false>(a, tiles, num_cus, s);
     return hipGetLastError();
   }
-  // class pairs: a workgroup per 16 columns while those fit the CUs three to
-  // each, else per 32
+  // class pairs; for long rows single classes, while a workgroup per segment
+  // fits the CUs (down, 40 blocks, with its tile launch: 18.8 -> 17.1 us at 5
+  // columns, 24.2 -> 21.0 at 21; Q/K/V and O, 10 and 8 blocks: 9.6 -> 9.7, 8.8 -> 9.1)
+  const bool single = a.total_tiles <= num_cus && a.nb >= 20;
+  if (!pair_out && single && l.cols <= 32) {
+    if (l.cols <= 16)
+      launch_mid_kernel<1, 1, false>(a, tiles, s);
+    else
+      launch_mid_kernel<2, 1, false>(a, tiles, s);
+    return hipGetLastError();
+  }
+  // a workgroup per 16 columns while those fit the CUs three to each (three
+  // groups of down 30.5 -> 25.1 us against two of 32), else per 32
   const bool narrow = l.cols <= 16 || (long long)a.total_tiles * ((l.cols + 15) / 16) <= 3 * num_cus;
   if (pair_out && narrow)
-    launch_mid_kernel<1, true>(a, tiles, s);
+    launch_mid_kernel<1, 2, true>(a, tiles, s);
   else if (pair_out)
-    launch_mid_kernel<2, true>(a, tiles, s);
+    launch_mid_kernel<2, 2, true>(a, tiles, s);
   else if (narrow)
-    launch_mid_kernel<1, false>(a, tiles, s);
+    launch_mid_kernel<1, 2, false>(a, tiles, s);
   else
-    launch_mid_kernel<2, false>(a, tiles, s);
+    launch_mid_kernel<2, 2, false>(a, tiles, s);
   return hipGetLastError();
 }
 
