@@ -199,11 +199,13 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const AttnArgs a, 
   // staging, the same for every thread (no branch, so no load waits on
   // another path's).  Values: 8 bytes (dims 4 v_dg .. + 3) of each of the
   // keys at V^T columns 8 v_q .. + 7 -- keys 4 v_q + i and 16 + 4 v_q + i --
-  // stored as four 16-byte column runs.  Keys: a quarter row of key k_j,
+  // stored as four 16-byte column runs (four lanes side by side take 32 bytes
+  // of one row: with a row per lane the L1's address unit was busy half the
+  // kernel's time).  Keys: a quarter row of key k_j,
   // 16-byte chunks k_e + 8 i, turned by 7 chunks on odd rows.  With the
   // padded strides each store's 8 (and 16) consecutive lanes then fill
   // distinct 16-byte slots of 128 (and 256) bytes.
-  const int v_q = tid & 3, v_dg = tid >> 2;   // columns 8 v_q.., dims 4 v_dg..
+  const int v_q = (tid >> 2) & 3, v_dg = (tid & 3) | ((tid >> 4) << 2);  // columns 8 v_q.., dims 4 v_dg..
   const int k_j = tid >> 3, k_e = tid & 7;    // key k_j, chunks (k_e + 8 i + 7 (k_j & 1)) % 32
   const int k_rot = k_e + 7 * (k_j & 1);
   uint2 vk[8];
@@ -212,22 +214,33 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const AttnArgs a, 
     const int slot = s0 + min(w, w_stop - 1);
     return slot >= cap ? slot - cap : slot;
   };
-  auto vrow = [&](int w) {
-    return reinterpret_cast<const uint2 *>(a.v_cache + head_base + (size_t)slot_of(w) * kHeadDim + 4 * v_dg);
+  // Byte offsets of a thread's rows from the tile's first slot.  A tile that
+  // neither passes w_stop nor wraps round the ring (all but one or two of a
+  // slice) takes them as they are; forming nine ring slots and addresses for
+  // every tile was a quarter of the loop's vector instructions.
+  constexpr uint32_t kRowBytes = 2 * kHeadDim;
+  const uint32_t v_at = (uint32_t)(4 * v_q) * kRowBytes + 8u * v_dg, k_at = (uint32_t)k_j * kRowBytes;
+  auto load = [&](int w0) {
+    const int s = slot_of(w0);  // the same for every thread
+    const uint8_t *vb = reinterpret_cast<const uint8_t *>(a.v_cache + head_base) + (size_t)s * kRowBytes;
+    const uint8_t *kb = reinterpret_cast<const uint8_t *>(a.k_cache + head_base) + (size_t)s * kRowBytes;
+    int vo[8], ko = (int)k_at;  // (negative past the ring's end)
+#pragma unroll
+    for (int i = 0; i < 8; i++) vo[i] = (int)(v_at + (uint32_t)((i & 3) + 16 * (i >> 2)) * kRowBytes);
+    if (w0 + kPfKeys > w_stop || s + kPfKeys > cap) {
+#pragma unroll
+      for (int i = 0; i < 8; i++)
+        vo[i] = (slot_of(w0 + 4 * v_q + (i & 3) + 16 * (i >> 2)) - s) * (int)kRowBytes + 8 * v_dg;
+      ko = (slot_of(w0 + k_j) - s) * (int)kRowBytes;
+    }
+#pragma unroll
+    for (int i = 0; i < 8; i++) vk[i] = *reinterpret_cast<const uint2 *>(vb + vo[i]);
+    const uint4 *kr = reinterpret_cast<const uint4 *>(kb + ko);
+    k0 = kr[k_rot & 31];
+    k1 = kr[(k_rot + 8) & 31];
+    k2 = kr[(k_rot + 16) & 31];
+    k3 = kr[(k_rot + 24) & 31];
   };
-  auto krow = [&](int w) {
-    return reinterpret_cast<const uint4 *>(a.k_cache + head_base + (size_t)slot_of(w) * kHeadDim);
-  };
-#define HP_PF_LOAD(w0)                                                                      \
-  do {                                                                                      \
-    _Pragma("unroll") for (int i = 0; i < 8; i++)                                           \
-        vk[i] = *vrow((w0) + 4 * v_q + (i & 3) + 16 * (i >> 2));                            \
-    const uint4 *kr = krow((w0) + k_j);                                                     \
-    k0 = kr[k_rot & 31];                                                                    \
-    k1 = kr[(k_rot + 8) & 31];                                                              \
-    k2 = kr[(k_rot + 16) & 31];                                                             \
-    k3 = kr[(k_rot + 24) & 31];                                                             \
-  } while (0)
 #define HP_PF_STORE(t)                                                                      \
   do {                                                                                      \
     _Pragma("unroll") for (int c = 0; c < 4; c++)                                           \
@@ -242,14 +255,14 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const AttnArgs a, 
   } while (0)
 
   if (w_begin < w_stop) {
-    HP_PF_LOAD(w_begin);
+    load(w_begin);
     HP_PF_STORE(sh[0]);
   }
   __syncthreads();
   int cur = 0;
   for (int w0 = w_begin; w0 < w_stop; w0 += kPfKeys, cur ^= 1) {
     const bool more = w0 + kPfKeys < w_stop;
-    if (more) HP_PF_LOAD(w0 + kPfKeys);  // the next tile streams in while this one computes
+    if (more) load(w0 + kPfKeys);  // the next tile streams in while this one computes
     const PfTile &t = sh[cur];
 
     // S^T of the 32 keys (two 16-key halves) x the wave's 16 query rows.
@@ -316,7 +329,6 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const AttnArgs a, 
     __syncthreads();
   }
 
-#undef HP_PF_LOAD
 #undef HP_PF_STORE
 // partials in attn_reduce_kernel's layout: chunk = this slice
   auto part_row = [&](int t, int h) {
