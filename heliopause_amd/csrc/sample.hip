@@ -16,7 +16,7 @@
 // the ones before it.  What bounds a column is the chain of its left-to-right
 // sums; each takes its terms from the lanes' registers (readlane), where one
 // lane reading them back from LDS paid an LDS round trip per term.  Five
-// columns of 40 candidates 34 -> 7 us, one 7 -> 6.
+// columns of 40 candidates 34 -> 10 us.
 #include "hp_common.h"
 #include "hp_exp.h"
 

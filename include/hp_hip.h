@@ -249,9 +249,10 @@ int32_t hp_hip_quantize_q8_k(const float *input, size_t input_len, size_t input_
 
 /* Matvec kernel selection (no counterpart in the reference; a tuning and
  * test hook): 0 = automatic (by column count and tile count: half-split
- * vector ALU for small projections, vector ALU for one column, matrix
- * cores for several columns of large ones, the bit-exact prefill kernel
- * from 32 columns, the fast prefill kernel from 64 on *_device calls), 1 = always the
+ * vector ALU for small projections, vector ALU for one column, the
+ * bit-exact mid kernels (matrix cores, every column of the launch) from five
+ * columns and from two of launches with many rows, the fast prefill kernel
+ * from 64 on *_device calls), 1 = always the
  * vector-ALU kernel, 2 = the matrix-core kernel whenever its LDS fits the
  * device, 3 = the half-split vector-ALU kernel (two lanes per row-block) for
  * up to four columns, 4 = the bit-exact prefill kernel (64-column tiles) for
