@@ -134,10 +134,18 @@ __device__ __forceinline__ int pf_seen(const PfWindow &w, int t_last) {
 
 constexpr int kXcds = 8;
 
+// Bytes of a K or V row in its ring, and the largest ring whose row offsets
+// fit 32 bits: in a tile that wraps round the ring's end they reach back by
+// almost the whole ring.  Larger rings take 64-bit offsets in every tile
+// (FAR; a kernel of its own, so that the others' tiles keep theirs).
+constexpr int kRowBytes = 2 * kHeadDim;
+constexpr int kNearSlots = 0x7FFFFFFF / kRowBytes;  // 4,194,303
+
 // Two workgroups per CU (the register budget then holds each wave to 256,
 // and two double-buffered tiles of 37 KB each fit the 160 KB of LDS): a
 // step waits on its next K/V tile's loads, and the other workgroup's waves
 // compute meanwhile.
+template <bool FAR>
 __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const AttnArgs a, int blocks, int items) {
   __shared__ __align__(16) PfTile sh[2];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -226,28 +234,30 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const AttnArgs a, 
     const int slot = s0 + min(w, w_stop - 1);
     return slot >= cap ? slot - cap : slot;
   };
-  // Byte offsets of a thread's rows from the tile's first slot.  A tile that
-  // neither passes w_stop nor wraps round the ring (all but one or two of a
-  // slice) takes them as they are; forming nine ring slots and addresses for
-  // every tile was a quarter of the loop's vector instructions.
-  constexpr uint32_t kRowBytes = 2 * kHeadDim;
-  const uint32_t v_at = (uint32_t)(4 * v_q) * kRowBytes + 8u * v_dg, k_at = (uint32_t)k_j * kRowBytes;
+  // A thread's rows from the tile's first slot, in bytes (FAR: in rows, made
+  // bytes in 64 bits at the load).  A tile that neither passes w_stop nor
+  // wraps round the ring (all but one or two of a slice) takes them as they
+  // are; forming nine ring slots and addresses for every tile was a quarter of
+  // the loop's vector instructions.
+  auto row_at = [&](int rows, int byte) { return FAR ? rows : rows * kRowBytes + byte; };
+  auto row_ptr = [&](const uint8_t *base, int at, int byte) {
+    return FAR ? base + (long long)at * kRowBytes + byte : base + at;
+  };
   auto load = [&](int w0) {
     const int s = slot_of(w0);  // the same for every thread
     const uint8_t *vb = reinterpret_cast<const uint8_t *>(a.v_cache + head_base) + (size_t)s * kRowBytes;
     const uint8_t *kb = reinterpret_cast<const uint8_t *>(a.k_cache + head_base) + (size_t)s * kRowBytes;
-    int vo[8], ko = (int)k_at;  // (negative past the ring's end)
+    int vo[8], ko = row_at(k_j, 0);  // (negative past the ring's end)
 #pragma unroll
-    for (int i = 0; i < 8; i++) vo[i] = (int)(v_at + (uint32_t)((i & 3) + 16 * (i >> 2)) * kRowBytes);
+    for (int i = 0; i < 8; i++) vo[i] = row_at(4 * v_q + (i & 3) + 16 * (i >> 2), 8 * v_dg);
     if (w0 + kPfKeys > w_stop || s + kPfKeys > cap) {
 #pragma unroll
-      for (int i = 0; i < 8; i++)
-        vo[i] = (slot_of(w0 + 4 * v_q + (i & 3) + 16 * (i >> 2)) - s) * (int)kRowBytes + 8 * v_dg;
-      ko = (slot_of(w0 + k_j) - s) * (int)kRowBytes;
+      for (int i = 0; i < 8; i++) vo[i] = row_at(slot_of(w0 + 4 * v_q + (i & 3) + 16 * (i >> 2)) - s, 8 * v_dg);
+      ko = row_at(slot_of(w0 + k_j) - s, 0);
     }
 #pragma unroll
-    for (int i = 0; i < 8; i++) vk[i] = *reinterpret_cast<const uint2 *>(vb + vo[i]);
-    const uint4 *kr = reinterpret_cast<const uint4 *>(kb + ko);
+    for (int i = 0; i < 8; i++) vk[i] = *reinterpret_cast<const uint2 *>(row_ptr(vb, vo[i], 8 * v_dg));
+    const uint4 *kr = reinterpret_cast<const uint4 *>(row_ptr(kb, ko, 0));
     k0 = kr[k_rot & 31];
     k1 = kr[(k_rot + 8) & 31];
     k2 = kr[(k_rot + 16) & 31];
@@ -467,7 +477,8 @@ hipError_t launch_attention_prefill(AttnArgs a, float *partials, int ranges, hip
   const int blocks = (a.tokens + Tq - 1) / Tq;
   const int items = blocks * a.nkv * ranges;
   const int per_xcd = (items + kXcds - 1) / kXcds;
-  hipLaunchKernelGGL(attn_prefill_kernel, dim3(per_xcd * kXcds), dim3(256), 0, s, a, blocks, items);
+  auto *k = a.capacity > kNearSlots ? attn_prefill_kernel<true> : attn_prefill_kernel<false>;
+  hipLaunchKernelGGL(k, dim3(per_xcd * kXcds), dim3(256), 0, s, a, blocks, items);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   const int tile_cols = a.o_tile_cols ? a.o_tile_cols : (a.tokens + kF2Cols - 1) / kF2Cols * kF2Cols;

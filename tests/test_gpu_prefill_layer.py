@@ -159,6 +159,37 @@ def test_prefill_attention(hip, D, tokens, nq, nkv, cap, pos, window, qscale):
     assert np.count_nonzero(steps) <= 0.02 * steps.size
 
 
+@pytest.mark.parametrize("cap", [4194303, 4194304, 4194400])
+def test_prefill_attention_wrap_of_large_ring(hip, D, cap):
+    """A window that wraps round the end of a ring whose row offsets (512
+    bytes a row, back by up to the whole ring) reach the largest 32-bit value,
+    and pass it: against the oracle over a 256-slot ring with the same keys."""
+    import torch
+
+    tokens, nq, window, small = 40, 2, 200, 256
+    pos = cap + 50
+    rng = np.random.default_rng(cap)
+    q = (rng.standard_normal((tokens, nq, 256)) * 0.25).astype(np.float32)
+    keys = np.arange(pos + tokens - window, pos + tokens)  # the window, cap - 110 to cap + 89
+    rows = rng.standard_normal((2, window, 256)).astype(np.float16)
+    rings = [torch.zeros(cap, 256, dtype=torch.int16, device="cuda:0") for _ in range(2)]
+    refs = np.zeros((2, 1, small, 256), np.float16)
+    for i in range(2):
+        rings[i][torch.from_numpy(keys % cap).to("cuda:0")] = _dev(rows[i].view(np.int16))
+        refs[i, 0, keys % small] = rows[i]
+    dq, dpos = _dev(q), _dev(np.array([pos], np.int32))
+    out = torch.empty(tokens * nq * 256, dtype=torch.float32, device="cuda:0")
+    print(f"prefill attention large ring cap={cap}", flush=True)
+    hip.gqa_attention_device(hip.attention_config(nq, 1, cap, sliding_window=window), dq.data_ptr(),
+                             rings[0].data_ptr(), rings[1].data_ptr(), dpos.data_ptr(), out.data_ptr(),
+                             token_count=tokens)
+    torch.cuda.synchronize()
+    got = out.cpu().numpy().reshape(tokens, nq, 256)
+    ref = D.decode_attention(q, refs[0], refs[1], pos, window)
+    assert max(_rel(got[t, h], ref[t, h]) for t in range(tokens) for h in range(nq)) <= 2.0 ** -8
+    assert np.count_nonzero(_f16_steps(got, ref)) <= 0.02 * got.size
+
+
 def test_prefill_attention_prep(hip, D):
     """Norms, RoPE and the cache append of 300 tokens (one launch)."""
     import torch
