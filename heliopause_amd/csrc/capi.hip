@@ -315,6 +315,7 @@ int cols_per_launch(const TileGeom &g, size_t max_lds) {
 // kernels, which read the weights once per 8 columns, are as fast.
 constexpr size_t kPrefillMinCols = 32;
 constexpr size_t kFastMinCols = 64;
+constexpr size_t kMaxTileCols = 65535;  // columns of one launch of the prefill and mid kernels
 
 // What the matrix-core kernels can take of a launch's weights: `tiles` all of
 // them (the tiles they address, below), `f16` also as single f16 operands (no
@@ -339,13 +340,15 @@ constexpr int kMidLargeSegs = 16;  // 16-row segments per CU
 // 0: not a prefill launch, 1: bit-exact prefill, 2: fast prefill
 // The automatic fast kernel takes every Q6_K weight (with full-range scales
 // as two exact operands, MfmaLaunch::wide6); the other prefill kernels, and
-// the forced fast one, take launches with single f16 operands only.
+// the forced fast one, take launches with single f16 operands only.  Launches
+// that are not for those run the vector-ALU kernels at any column count.
 int chunk_kind(size_t cols, MfmaFit fit) {
   const State &s = st();
   const int forced = s.matvec_kernel;
   if (!fit.tiles) return 0;
   if (!fit.f16) {
-    const bool fast = forced == 0 && cols >= kFastMinCols && !s.host_exact && prefill_fast_lds_bytes() <= s.max_lds;
+    const bool fast = forced == 0 && cols >= kFastMinCols && cols <= kMaxTileCols && !s.host_exact &&
+                      prefill_fast_lds_bytes() <= s.max_lds;
     return fast ? 2 : 0;
   }
   const bool exact_fits = prefill_lds_bytes() <= s.max_lds;
@@ -365,7 +368,7 @@ int prefill_kind(size_t cols, MfmaFit fit) {
   const State &s = st();
   const int kind = chunk_kind(cols, fit);
   const size_t least = fit.segs >= (long long)kMidLargeSegs * s.num_cus ? kMidMinColsLarge : kMidMinCols;
-  if (s.matvec_kernel == 0 && kind != 2 && fit.tiles && cols >= least && cols <= 65535 && mid_lds_bytes() <= s.max_lds)
+  if (s.matvec_kernel == 0 && kind != 2 && fit.tiles && cols >= least && cols <= kMaxTileCols && mid_lds_bytes() <= s.max_lds)
     return 3;
   return kind;
 }
@@ -538,7 +541,7 @@ int32_t run_matvec(size_t count, Handle *const *hs, const float *d_input, size_t
   const bool image_ok = s.images && cols >= 2 && image_input_ok(count, hs, cols, kind);
   const bool wide = kind == 0 && use_wide(count, hs, cols);
   const bool wide_norm = wide && cols == 1 && g_nb_of(hs) <= 16;  // the wide kernel's norm prologue
-  if (kind && cols > 65535) return fail(HP_ERR_SHAPE, "too many columns");
+  if (kind && cols > kMaxTileCols) return fail(HP_ERR_SHAPE, "too many columns");
   // a deferred GeGLU tail is completed by the fast prefill kernel's pre-pass
   if (tail_in && (kind != 2 || norm || tiles_in)) return fail(HP_ERR_ARG, "deferred GeGLU tail needs the fast prefill");
   MfmaLaunch l{};

@@ -86,6 +86,28 @@ def test_fast_prefill_full_range(hip, oracle, layouts, rows, k, m):
         assert np.max(np.abs(g - ref4.reshape(-1))) <= 1e-4 * np.abs(ref4).max()
 
 
+def test_full_range_more_columns_than_a_prefill_launch(hip, oracle):
+    """65,537 columns on the device: more than one launch of the prefill
+    kernels takes, so the vector-ALU kernels run (the oracle's bits)."""
+    import torch
+
+    rows, k, m = 16, 256, 65537
+    print(f"full range m={m}", flush=True)
+    seed = S.derive(S.BASE_SEED, "full-range-many")
+    w, part = _full_range(seed, rows, k), S.activations(seed, 64, k)
+    x = np.resize(part, (m, k))  # column c is part[c % 64]
+    h = hip.createHipQuantizedWeightHandle("Q6_K", w, k, rows)
+    try:
+        dx, out = _device(x.reshape(-1)), torch.empty(rows * m, dtype=torch.float32, device="cuda:0")
+        hip.matmul_multi_device([h.handle], dx.data_ptr(), k, m, [out.data_ptr()], [out.numel()])
+        torch.cuda.synchronize()
+        got = out.cpu().numpy().reshape(m, rows)
+    finally:
+        hip.releaseHipQuantizedWeightHandle(h)
+    ref = oracle.matmul(3, w, part, rows).reshape(64, rows)
+    assert np.array_equal(got.view(np.uint32), np.resize(ref, (m, rows)).view(np.uint32))
+
+
 def test_fast_prefill_full_range_geglu(hip, oracle, layouts):
     """gate and up as full-range Q6_K in one tile, GeGLU in its epilogue:
     elements within two f16 steps (gelu rounds its input and result to f16),
