@@ -228,18 +228,29 @@ int32_t grow(void **p, size_t *cap, size_t bytes) {
 
 // Scratch of `kind` for work queued on `stream` (hp_scratch.h): per stream,
 // grow-only, and never grown while the stream captures a graph.
-int32_t stream_scratch(hipStream_t stream, int kind, size_t bytes, void **out, bool zero = false) {
+int scratch_status(hipStream_t stream, int kind, size_t bytes, void **out, bool zero) {
   State &s = st();
   void *key = stream ? static_cast<void *>(stream) : static_cast<void *>(s.stream);
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(stream, &cs) != hipSuccess) cs = hipStreamCaptureStatusNone;
-  switch (s.pool.get(key, kind, bytes, cs != hipStreamCaptureStatusNone, zero, out)) {
+  return s.pool.get(key, kind, bytes, cs != hipStreamCaptureStatusNone, zero, out);
+}
+
+int32_t stream_scratch(hipStream_t stream, int kind, size_t bytes, void **out, bool zero = false) {
+  switch (scratch_status(stream, kind, bytes, out, zero)) {
     case kScratchOk: return HP_OK;
     case kScratchCapturing:
       return fail(HP_ERR_ARG, "scratch must be sized by an uncaptured call of this shape before graph capture");
     case kScratchZeroFailed: return fail(HP_ERR_HIP, "clearing scratch failed");
     default: return fail(HP_ERR_OOM, "device allocation failed");
   }
+}
+
+// The same for a launch that can do without: null when there is none, which
+// is no error of the call (its last-error text stays as it was).
+uint8_t *try_scratch(hipStream_t stream, int kind, size_t bytes) {
+  void *p = nullptr;
+  return scratch_status(stream, kind, bytes, &p, false) == kScratchOk ? static_cast<uint8_t *>(p) : nullptr;
 }
 
 hipEvent_t take_event() {
@@ -489,9 +500,7 @@ int32_t run_norm(const float *y, int rows, int n, const float *w_post, const flo
 
 // Scratch for the mid kernel's activation tiles, or null when there is none.
 uint8_t *mid_scratch(size_t input_size, size_t cols, hipStream_t stream) {
-  void *p = nullptr;
-  const int32_t rc = stream_scratch(stream, kScratchPrefill, mid_bytes((int)input_size, (int)cols), &p);
-  return rc == HP_OK ? static_cast<uint8_t *>(p) : nullptr;
+  return try_scratch(stream, kScratchPrefill, mid_bytes((int)input_size, (int)cols));
 }
 
 // Whether a one-column launch over these weights runs a vector-ALU kernel,

@@ -138,3 +138,33 @@ def test_capture_without_scratch(hip, oracle):
     finally:
         hip.releaseHipQuantizedWeightHandle(h)
         hip.lib().hp_hip_release_stream_scratch(ctypes.c_void_p(stream.cuda_stream))
+
+
+def test_capture_without_scratch_leaves_no_error(hip, oracle):
+    """A call that runs other kernels for want of scratch has succeeded: the
+    last-error text is still that of the last call that failed."""
+    import torch
+
+    rows, k, m = 64, 768, 8
+    w, x = _blocks("Q6_K", 5, rows, k), S.activations(6, m, k)
+    h = hip.createHipQuantizedWeightHandle("Q6_K", w, k, rows)
+    stream = torch.cuda.Stream()
+    try:
+        dx, out = torch.from_numpy(x.reshape(-1)).to("cuda:0"), torch.empty(rows * m, device="cuda:0")
+        torch.cuda.synchronize()
+        with pytest.raises(Exception):
+            hip.matmul_multi_device([h.handle], dx.data_ptr(), k, m, [out.data_ptr()], [out.numel() - 1])
+        failed = hip.last_error()
+        assert failed
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            hip.matmul_multi_device([h.handle], dx.data_ptr(), k, m, [out.data_ptr()], [out.numel()],
+                                    stream.cuda_stream)
+        assert hip.last_error() == failed
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(_bits(out.cpu().numpy()), _bits(oracle.matmul(3, w, x, rows)))
+        del graph
+    finally:
+        hip.releaseHipQuantizedWeightHandle(h)
+        hip.lib().hp_hip_release_stream_scratch(ctypes.c_void_p(stream.cuda_stream))
