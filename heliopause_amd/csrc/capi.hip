@@ -570,10 +570,17 @@ int32_t run_matvec(size_t count, Handle *const *hs, const float *d_input, size_t
   l.wide6 = !fit.f16;
   if (kind && !pre) {
     const size_t need = kind == 2 ? prefill_fast_bytes(l, s.num_cus) : prefill_q8k_bytes((int)input_size, (int)cols);
-    void *p = nullptr;
-    int32_t rc = stream_scratch(stream, kScratchPrefill, need, &p);
-    if (rc != HP_OK) return rc;
-    pre = static_cast<uint8_t *>(p);
+    if (kind == 2 && !fit.f16 && !tail_in && !tiles_in) {
+      // full-range weights without scratch (a captured call that no earlier
+      // call has sized it for): the vector-ALU kernels, which need none
+      pre = try_scratch(stream, kScratchPrefill, need);
+      if (!pre) kind = 0;
+    } else {
+      void *p = nullptr;
+      int32_t rc = stream_scratch(stream, kScratchPrefill, need, &p);
+      if (rc != HP_OK) return rc;
+      pre = static_cast<uint8_t *>(p);
+    }
   }
   // the norm kernel below, or the producer of d_input (tiles_in: the prefill
   // attention's slice merge), wrote the fast prefill's tiles

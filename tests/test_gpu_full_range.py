@@ -7,6 +7,8 @@ the exact integers with the rounding bound of its f32 tail: per block three
 roundings (dw * D, times dx, the running sum; each at most 2^-24 of the terms
 so far), block ranges add one more each, so (3 nb + 8) 2^-24 sum_b |t_b|.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -106,6 +108,49 @@ def test_full_range_more_columns_than_a_prefill_launch(hip, oracle):
         hip.releaseHipQuantizedWeightHandle(h)
     ref = oracle.matmul(3, w, part, rows).reshape(64, rows)
     assert np.array_equal(got.view(np.uint32), np.resize(ref, (m, rows)).view(np.uint32))
+
+
+def test_full_range_capture_without_scratch(hip, oracle):
+    """A captured call of 70 columns on a stream that no call has sized scratch
+    for is accepted (the vector-ALU kernels: the oracle's bits on every
+    replay); sized, the capture takes the fast prefill kernel."""
+    import torch
+
+    rows, k, m = 40, 768, 70
+    seed = S.derive(S.BASE_SEED, "full-range-capture")
+    w, x = _full_range(seed, rows, k), S.activations(seed, m, k)
+    ref = oracle.matmul(3, w, x, rows)
+    t = _terms(oracle, w, x, rows)
+    bound = (3 * (k // 256) + 8) * 2.0 ** -24 * np.abs(t).sum(2)
+    h = hip.createHipQuantizedWeightHandle("Q6_K", w, k, rows)
+    stream = torch.cuda.Stream()
+    print("full range capture", flush=True)
+    try:
+        dx, out = _device(x.reshape(-1)), torch.empty(rows * m, dtype=torch.float32, device="cuda:0")
+        torch.cuda.synchronize()
+        run = lambda: hip.matmul_multi_device([h.handle], dx.data_ptr(), k, m, [out.data_ptr()],  # noqa: E731
+                                              [out.numel()], stream.cuda_stream)
+        for sized in (False, True):
+            if sized:
+                run()
+                torch.cuda.synchronize()
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph, stream=stream):
+                run()
+            for _ in range(3):
+                out.zero_()
+                torch.cuda.synchronize()
+                graph.replay()
+                torch.cuda.synchronize()
+                got = out.cpu().numpy()
+                if sized:
+                    assert np.all(np.abs(got.reshape(m, rows).T.astype(np.float64) - t.sum(2)) <= bound)
+                else:
+                    assert np.array_equal(got.view(np.uint32), ref.reshape(-1).view(np.uint32))
+            del graph
+    finally:
+        hip.releaseHipQuantizedWeightHandle(h)
+        hip.lib().hp_hip_release_stream_scratch(ctypes.c_void_p(stream.cuda_stream))
 
 
 def test_fast_prefill_full_range_geglu(hip, oracle, layouts):
