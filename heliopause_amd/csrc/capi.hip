@@ -62,9 +62,19 @@ struct ProfileSlot {
   uint64_t launches = 0;
 };
 
+// hipMalloc, whose failure is the return value only: the runtime's last error
+// is cleared, or the launches of the next call, which end with
+// hipGetLastError, would report it as their own.
+bool dev_malloc(void **p, size_t bytes) {
+  if (hipMalloc(p, bytes) == hipSuccess) return true;
+  (void)hipGetLastError();
+  *p = nullptr;
+  return false;
+}
+
 // Device memory for the scratch pool (hp_scratch.h).
 struct HipAlloc {
-  bool alloc(void **p, size_t bytes) { return hipMalloc(p, bytes) == hipSuccess; }
+  bool alloc(void **p, size_t bytes) { return dev_malloc(p, bytes); }
   void free(void *p) { (void)hipFree(p); }
   bool zero(void *p, size_t bytes, void *stream) {
     hipStream_t q = static_cast<hipStream_t>(stream);
@@ -187,7 +197,7 @@ int32_t ensure_init(int device) {
   if (!sym) return fail(HP_ERR_HIP, "hipGetSymbolAddress(scratch) returned null");
   s.static_scratch = static_cast<uint8_t *>(sym);
   // the gelu table of the GeGLU launches (hp_gelu.h gelu_lut), built once
-  if (hipMalloc((void **)&s.gelu_lut, 65536 * sizeof(uint16_t)) != hipSuccess) {
+  if (!dev_malloc((void **)&s.gelu_lut, 65536 * sizeof(uint16_t))) {
     s.gelu_lut = nullptr;
     return fail(HP_ERR_OOM, "gelu table allocation failed");
   }
@@ -218,7 +228,7 @@ int32_t grow(void **p, size_t *cap, size_t bytes) {
     *cap = 0;
   }
   size_t want = bytes < 4096 ? 4096 : bytes;
-  if (hipMalloc(p, want) != hipSuccess) {
+  if (!dev_malloc(p, want)) {
     *p = nullptr;
     return fail(HP_ERR_OOM, "device allocation failed");
   }
@@ -958,7 +968,7 @@ int32_t upload_common(int32_t type_id, const void *src, bool src_device, size_t 
   const int nb = (int)(input_size / kQK);
   const size_t tile_bytes = (weight_len + 255) & ~(size_t)255;
   h.seg_bytes = s.both_layouts ? mfma_segment_bytes(type_id, (int)row_count, nb) : 0;
-  if (hipMalloc((void **)&h.data, tile_bytes + h.seg_bytes + 256) != hipSuccess)
+  if (!dev_malloc((void **)&h.data, tile_bytes + h.seg_bytes + 256))
     return fail(HP_ERR_OOM, "weight allocation failed");
   if (s.both_layouts) h.segs = h.data + tile_bytes;
   h.f16_flag = reinterpret_cast<uint32_t *>(h.data + tile_bytes + h.seg_bytes);
@@ -968,7 +978,7 @@ int32_t upload_common(int32_t type_id, const void *src, bool src_device, size_t 
   const uint8_t *raw = static_cast<const uint8_t *>(src);
   uint8_t *staging = nullptr;
   if (!src_device) {
-    if (hipMalloc((void **)&staging, weight_len) != hipSuccess) {
+    if (!dev_malloc((void **)&staging, weight_len)) {
       (void)hipFree(h.data);
       return fail(HP_ERR_OOM, "staging allocation failed");
     }
@@ -1518,7 +1528,7 @@ int32_t fused_table(const std::vector<FusedLayer> &layers, hipStream_t stream, c
   if (cs != hipStreamCaptureStatusNone)
     return fail(HP_ERR_ARG, "decode layers: a captured call must follow an uncaptured call with the same layers");
   void *d = nullptr;
-  if (hipMalloc(&d, bytes.size()) != hipSuccess) return fail(HP_ERR_OOM, "device allocation failed");
+  if (!dev_malloc(&d, bytes.size())) return fail(HP_ERR_OOM, "device allocation failed");
   if (hipMemcpyAsync(d, bytes.data(), bytes.size(), hipMemcpyHostToDevice, stream) != hipSuccess ||
       hipStreamSynchronize(stream) != hipSuccess) {
     (void)hipFree(d);
@@ -1858,7 +1868,7 @@ int32_t hp_hip_dequantize(uint64_t handle, size_t row_start, size_t row_count, f
     return fail(HP_ERR_SHAPE, "dequantize range mismatch");
   if (row_count == 0) return HP_OK;
   float *d = nullptr;
-  if (hipMalloc((void **)&d, output_len * sizeof(float)) != hipSuccess) return fail(HP_ERR_OOM, "dequant buffer");
+  if (!dev_malloc((void **)&d, output_len * sizeof(float))) return fail(HP_ERR_OOM, "dequant buffer");
   hipError_t e = launch_dequantize(h->type, h->data, h->dplane, (int)h->row_count, h->g, (int)row_start,
                                    (int)row_count, d, s.stream);
   if (e == hipSuccess) e = hipMemcpyAsync(output, d, output_len * sizeof(float), hipMemcpyDeviceToHost, s.stream);
@@ -2115,10 +2125,7 @@ int32_t hp_hip_device_alloc(size_t bytes, void **d_out) {
   HP_HIP_TRY(hipStreamIsCapturing(s.stream, &cs));
   if (cs != hipStreamCaptureStatusNone) return fail(HP_ERR_ARG, "no allocation while the library stream captures");
   void *p = nullptr;
-  if (hipMalloc(&p, bytes) != hipSuccess) {
-    (void)hipGetLastError();
-    return fail(HP_ERR_OOM, "device allocation failed");
-  }
+  if (!dev_malloc(&p, bytes)) return fail(HP_ERR_OOM, "device allocation failed");
   if (hipMemsetAsync(p, 0, bytes, s.stream) != hipSuccess || hipStreamSynchronize(s.stream) != hipSuccess) {
     (void)hipFree(p);
     return fail(HP_ERR_HIP, "device allocation could not be cleared");
@@ -2252,7 +2259,7 @@ int32_t hp_hip_quantize_q8_k(const float *input, size_t input_len, size_t input_
   const size_t nb = input_size / kQK;
   uint8_t *buf = nullptr;
   const size_t bytes = input_len * 4 + input_len + column_count * nb * 4 + input_len / 32 * 2;
-  if (hipMalloc((void **)&buf, bytes) != hipSuccess) return fail(HP_ERR_OOM, "q8_k buffer");
+  if (!dev_malloc((void **)&buf, bytes)) return fail(HP_ERR_OOM, "q8_k buffer");
   float *dx = reinterpret_cast<float *>(buf);
   int8_t *dq = reinterpret_cast<int8_t *>(buf + input_len * 4);
   float *dd = reinterpret_cast<float *>(buf + input_len * 5);

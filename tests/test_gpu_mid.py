@@ -168,3 +168,25 @@ def test_capture_without_scratch_leaves_no_error(hip, oracle):
     finally:
         hip.releaseHipQuantizedWeightHandle(h)
         hip.lib().hp_hip_release_stream_scratch(ctypes.c_void_p(stream.cuda_stream))
+
+
+def test_failed_allocation_is_not_the_next_calls_error(hip, oracle):
+    """Every allocation of the library, scratch among them, goes through one
+    function.  After one has failed (a weight of 600 GB: refused before its
+    bytes are read), the launches of the next call still succeed."""
+    import torch
+
+    rows, k, m = 32, 512, 9
+    w, x = _blocks("Q4_K", 7, rows, k), S.activations(8, m, k)
+    h = hip.createHipQuantizedWeightHandle("Q4_K", w, k, rows)
+    try:
+        small = torch.zeros(256, dtype=torch.uint8, device="cuda:0")
+        big_k, big_rows = 1 << 20, 1 << 20
+        out = ctypes.c_uint64(0)
+        code = hip.lib().hp_hip_weight_upload_device(TYPES["Q4_K"], small.data_ptr(), big_k // 256 * 144 * big_rows,
+                                                     big_k, big_rows, ctypes.byref(out))
+        assert code != 0 and "allocation" in hip.last_error()
+        got = hip.matMulQuantizedHipResident(h, x, k, rows, m)
+        assert np.array_equal(_bits(got), _bits(oracle.matmul(1, w, x, rows)))
+    finally:
+        hip.releaseHipQuantizedWeightHandle(h)
