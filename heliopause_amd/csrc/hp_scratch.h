@@ -16,7 +16,9 @@
 //     never otherwise.  Growth itself is refused while the stream is
 //     capturing (the allocation would not be part of the graph), so a
 //     captured call must follow an uncaptured call of the same shape.
-// Capacities grow at least 2x, so retired memory stays below the live size.
+// Capacities grow at least 2x, so retired memory stays below the live size
+// (where memory allows: a device that cannot give twice the old capacity is
+// asked for the size of the call).
 //
 // Host-only C++ with the allocator as a template parameter, so the policy
 // can be exercised on the CPU with a recording allocator.
@@ -69,10 +71,15 @@ class ScratchPool {
       return kScratchOk;
     }
     if (capturing) return kScratchCapturing;
-    size_t want = bytes < 4096 ? 4096 : bytes;
-    if (b.p && want < 2 * b.cap) want = 2 * b.cap;
+    const size_t least = bytes < 4096 ? 4096 : bytes;
+    size_t want = b.p && least < 2 * b.cap ? 2 * b.cap : least;
     void *p = nullptr;
-    if (!alloc_.alloc(&p, want) || !p) return kScratchNoMemory;
+    if (!alloc_.alloc(&p, want) || !p) {
+      if (want == least) return kScratchNoMemory;
+      want = least;
+      p = nullptr;
+      if (!alloc_.alloc(&p, want) || !p) return kScratchNoMemory;
+    }
     if (zero && !alloc_.zero(p, want, stream)) {
       alloc_.free(p);
       return kScratchZeroFailed;

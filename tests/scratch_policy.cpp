@@ -98,6 +98,19 @@ int main() {
   check(pool.get(s2, hp::kScratchDecode, 1 << 20, false, false, &f) == hp::kScratchNoMemory, "allocation failure");
   check(pool.get(s2, hp::kScratchDecode, 100, false, false, &f) == hp::kScratchOk && f == d, "old buffer kept");
   check(rec.frees == 0, "still no free before release_all");
+  // growth of less than twice falls back to the size asked for, once
+  {
+    Pool own;
+    void *a = nullptr, *b = nullptr;
+    check(own.get(s1, hp::kScratchDecode, 8192, false, false, &a) == hp::kScratchOk, "first buffer");
+    rec.fail_next = true;
+    check(own.get(s1, hp::kScratchDecode, 10000, false, false, &b) == hp::kScratchOk && b != a, "exact size");
+    check(own.stats().live_bytes == 10000 && own.stats().retired_bytes == 8192, "exact size counted");
+    check(own.get(s1, hp::kScratchDecode, 10001, false, false, &b) == hp::kScratchOk, "growth again");
+    check(own.stats().live_bytes == 20000, "doubled again");
+    own.release_all();
+    rec.frees = 0;
+  }
   // releasing one stream frees its live and retired buffers only
   void *s3 = reinterpret_cast<void *>(0x3000), *g1 = nullptr, *g2 = nullptr;
   check(pool.get(s3, hp::kScratchDecode, 5000, false, false, &g1) == hp::kScratchOk, "third stream");
