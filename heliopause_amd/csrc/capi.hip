@@ -10,6 +10,7 @@
 #include "../../include/hp_hip.h"
 #include "hp_common.h"
 #include "hp_fused.h"
+#include "hp_mid_policy.h"
 #include "hp_scratch.h"
 
 #include <algorithm>
@@ -341,22 +342,9 @@ constexpr size_t kMaxTileCols = 65535;  // columns of one launch of the prefill 
 // What the matrix-core kernels can take of a launch's weights: `tiles` all of
 // them (the tiles they address, below), `f16` also as single f16 operands (no
 // Q6_K weight with scales beyond those, Handle::f16_exact).
-struct MfmaFit {
-  bool tiles, f16;
-  long long segs;  // the launch's 16-row segments
+struct MfmaFit : MidShape {
+  bool tiles;
 };
-
-// The mid kernels (kquant_mid.hip): every column of a launch on the matrix
-// cores, bit-exact.  They take the column counts below the fast kernel's, and
-// every count of the host-pointer calls: from five columns on (measured against
-// the vector-ALU and kquant_mfma kernels: five columns of Q/K/V 14.3 -> 9.5 us,
-// of the FFN 61.8 -> 36.0; at four O 6.9 -> 9.1, Q/K/V 9.8 -> 9.8, with the
-// launch that writes the activation tiles), and from two on for launches of 16
-// segments a CU (the head, two columns 176 -> 155 us, three 223 -> 164; heads
-// of 2000 segments the same either way).
-constexpr size_t kMidMinCols = 5;
-constexpr size_t kMidMinColsLarge = 2;
-constexpr int kMidLargeSegs = 16;  // 16-row segments per CU
 
 // 0: not a prefill launch, 1: bit-exact prefill, 2: fast prefill
 // The automatic fast kernel takes every Q6_K weight (with full-range scales
@@ -382,14 +370,17 @@ int chunk_kind(size_t cols, MfmaFit fit) {
   return 0;
 }
 
-// The same, or 3: the mid kernel.  A launch whose activation tiles cannot be
-// had (a captured call that no earlier call has sized scratch for, which the
-// kernels of chunk_kind 0 do not need) runs as chunk_kind says: the same bits.
+// The same, or 3: the mid kernels (kquant_mid.hip; every column of a launch on
+// the matrix cores, bit-exact) for the launches of hp_mid_policy.h below the
+// fast kernel's column counts, and at every count of the host-pointer calls.
+// A launch whose activation tiles cannot be had (a captured call that no
+// earlier call has sized scratch for, which the kernels of chunk_kind 0 do not
+// need) runs as chunk_kind says: the same bits.
 int prefill_kind(size_t cols, MfmaFit fit) {
   const State &s = st();
   const int kind = chunk_kind(cols, fit);
-  const size_t least = fit.segs >= (long long)kMidLargeSegs * s.num_cus ? kMidMinColsLarge : kMidMinCols;
-  if (s.matvec_kernel == 0 && kind != 2 && fit.tiles && cols >= least && cols <= kMaxTileCols && mid_lds_bytes() <= s.max_lds)
+  if (s.matvec_kernel == 0 && kind != 2 && fit.tiles && cols <= kMaxTileCols && mid_lds_bytes() <= s.max_lds &&
+      mid_takes(fit, cols))
     return 3;
   return kind;
 }
@@ -441,12 +432,16 @@ int g_nb_of(Handle *const *hs) { return hs[0]->g.nb; }
 // matrix-core kernels' 32-bit tile offsets (under 4 GiB).
 MfmaFit mfma_fit(size_t count, Handle *const *hs) {
   bool tiles = false;
-  MfmaFit f{true, true, 0};
+  MfmaFit f{};
+  f.tiles = f.f16 = true;
+  f.nb = hs[0]->g.nb;
+  f.cus = st().num_cus;
   for (size_t i = 0; i < count; i++) tiles = tiles || !hs[i]->segs;
   for (size_t i = 0; i < count; i++) {
     if (tiles && hs[i]->byte_length >= ((size_t)1 << 32)) f.tiles = f.f16 = false;
     if (!hs[i]->f16_exact) f.f16 = false;
     f.segs += (long long)((hs[i]->row_count + 15) / 16);
+    (hs[i]->type == kTypeQ4K ? f.q4 : f.q6) = true;
   }
   return f;
 }

@@ -27,6 +27,7 @@
 #include "hp_f2tile.h"
 #include "hp_gelu.h"
 #include "hp_mfma.h"
+#include "hp_mid_policy.h"
 #include "hp_wfrag.h"
 
 namespace hp {
@@ -812,9 +813,10 @@ hipError_t launch_mid(const MfmaLaunch &l, const uint8_t *xt, const uint16_t *ge
   a.gelu_lut = gelu_lut;
   const bool tiles = launch_reads_tiles(l);
   // row waves from two segments of one type a CU on
-  bool one_type = true;
-  for (int i = 1; i < l.count; i++) one_type = one_type && l.type[i] == l.type[0];
-  if (one_type && a.total_tiles >= 2 * num_cus) {
+  MidShape shape{a.total_tiles, a.nb, false, false, !l.wide6, num_cus};
+  for (int i = 0; i < l.count; i++) (l.type[i] == kTypeQ4K ? shape.q4 : shape.q6) = true;
+  if (!mid_grid_fits(shape, l.cols)) return hipErrorInvalidValue;
+  if (mid_row_waves(shape)) {
     if (pair_out && l.cols <= 16)
       launch_rows_kernel<1, true>(a, tiles, num_cus, s);
     else if (pair_out)
