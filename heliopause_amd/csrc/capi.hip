@@ -745,7 +745,8 @@ int32_t run_matvec_geglu(Handle *hg, Handle *hu, const float *d_input, size_t in
   const TileGeom g = hg->g;
   const int tiles16 = 2 * (int)((rows + 15) / 16);
   Handle *pair[2] = {hg, hu};
-  const MfmaFit fit = mfma_fit(2, pair);
+  MfmaFit fit = mfma_fit(2, pair);
+  fit.pair = true;
   int kind = prefill_kind(cols, fit);
   uint8_t *pre = nullptr;  // the prefill kernels' scratch, tiles first
   if (kind == 3) {

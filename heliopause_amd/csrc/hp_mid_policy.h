@@ -15,17 +15,15 @@ struct MidShape {
   int nb;          // blocks of a row
   bool q4, q6;     // some weight is Q4_K, Q6_K
   bool f16;        // every weight is exact in single f16 operands (no full-range Q6_K scales)
+  bool pair;       // gate and up with their GeGLU
   int cus;
 };
 
 // From five columns on (measured against the vector-ALU and kquant_mfma
 // kernels: five columns of Q/K/V 14.3 -> 9.5 us, of the FFN 61.8 -> 36.0; at
 // four O 6.9 -> 9.1, Q/K/V 9.8 -> 9.8, with the launch that writes the
-// activation tiles), and from two on for launches of 16 segments a CU (the
-// head, two columns 176 -> 155 us, three 223 -> 164; heads of 2000 segments
-// the same either way).
+// activation tiles), and from two on for some launches of 16 segments a CU.
 constexpr size_t kMidMinCols = 5;
-constexpr size_t kMidMinColsLarge = 2;
 constexpr int kMidLargeSegs = 16;  // 16-row segments per CU
 
 // Row waves (a wave per segment) or else class pairs.
@@ -39,9 +37,40 @@ inline bool mid_grid_fits(const MidShape &l, size_t cols) {
   return mid_row_waves(l) || (unsigned long long)((l.segs + 7) / 8 * 8) * groups < (1ull << 32) / 512;
 }
 
+// Row waves' items of eight segments, one workgroup a CU: the last round of
+// items at least leaves no more than a fifth of the launch's CU time idle.
+inline bool mid_rounds_full(const MidShape &l) {
+  const long long items = (l.segs + 7) / 8, rounds = (items + l.cus - 1) / l.cus;
+  return 5 * items >= 4 * rounds * l.cus;
+}
+
+// Two to four columns of a launch of 16 segments a CU (heads; gate/up of
+// 32768 rows).  Times are this kernel's over the other's, measured at 65536 to
+// 262144 rows (gate/up: 32768 to 65536) of 1, 4, 10 and 15 blocks.
+inline bool mid_takes_few(const MidShape &l, size_t cols) {
+  if (cols < 2 || l.segs < (long long)kMidLargeSegs * l.cus) return false;
+  // mixed types, class pairs: full-range Q6_K from 10 blocks 0.70 to 0.87 at
+  // three and four columns; else 0.87 to 1.58
+  if (!mid_row_waves(l)) return !l.f16 && l.nb >= 10 && cols > 2;
+  if (l.pair) {
+    // the wide kernel with GeGLU: four columns 0.35 to 0.97; three 0.54 to
+    // 1.03 for Q6_K, 0.63 to 0.72 for Q4_K from 10 blocks (fewer: up to
+    // 1.22); two 0.67 to 0.86 for Q6_K from 10 blocks (fewer: up to 1.18),
+    // 0.76 to 0.96 for Q4_K from 15 (10 blocks: up to 1.15)
+    if (cols == 4) return true;
+    if (cols == 3) return !l.q4 || l.nb >= 10;
+    return l.nb >= (l.q4 ? 15 : 10);
+  }
+  // kquant_mfma, one launch and one operand a weight: 0.93 to 1.46, Q6_K 1.03 and more
+  if (l.f16) return false;
+  // the vector-ALU kernels, weights read once for the columns they hold: from
+  // four blocks 0.56 to 0.90 at three and four columns, 0.80 to 1.02 at two
+  // (last round nearly empty: 1.05); one block up to 1.48
+  return l.nb >= 4 && (cols > 2 || mid_rounds_full(l));
+}
+
 inline bool mid_takes(const MidShape &l, size_t cols) {
-  const size_t least = l.segs >= (long long)kMidLargeSegs * l.cus ? kMidMinColsLarge : kMidMinCols;
-  return cols >= least && mid_grid_fits(l, cols);
+  return mid_grid_fits(l, cols) && (cols >= kMidMinCols || mid_takes_few(l, cols));
 }
 
 }  // namespace hp

@@ -813,7 +813,9 @@ hipError_t launch_mid(const MfmaLaunch &l, const uint8_t *xt, const uint16_t *ge
   a.gelu_lut = gelu_lut;
   const bool tiles = launch_reads_tiles(l);
   // row waves from two segments of one type a CU on
-  MidShape shape{a.total_tiles, a.nb, false, false, !l.wide6, num_cus};
+  MidShape shape{};
+  shape.segs = a.total_tiles;
+  shape.cus = num_cus;
   for (int i = 0; i < l.count; i++) (l.type[i] == kTypeQ4K ? shape.q4 : shape.q6) = true;
   if (!mid_grid_fits(shape, l.cols)) return hipErrorInvalidValue;
   if (mid_row_waves(shape)) {

@@ -2,13 +2,21 @@
 // 256 CUs.
 #include <cstdio>
 #include <cstdlib>
+#include <initializer_list>
 
 #include "hp_mid_policy.h"
 
 namespace {
 
 hp::MidShape shape(long long rows, int k, bool q4, bool q6, bool f16) {
-  return hp::MidShape{(rows + 15) / 16, k / 256, q4, q6, f16, 256};
+  hp::MidShape l{};
+  l.segs = (rows + 15) / 16;
+  l.nb = k / 256;
+  l.q4 = q4;
+  l.q6 = q6;
+  l.f16 = f16;
+  l.cus = 256;
+  return l;
 }
 
 int failures = 0;
@@ -33,10 +41,36 @@ void grids() {
   check(hp::mid_takes(shape(262144, 2560, false, true, false), 65535), "one type: row waves");
 }
 
+// Two to four columns: single-operand launches keep kquant_mfma; full-range
+// Q6_K from four blocks, at two columns with full rounds only; gate/up by type
+// and row length; small launches never.
+void few_columns() {
+  for (size_t cols = 2; cols <= 4; cols++) {
+    for (int k : {256, 1024, 2560, 3840}) {
+      check(!hp::mid_takes(shape(262144, k, true, false, true), cols), "Q4_K head");
+      check(!hp::mid_takes(shape(262144, k, false, true, true), cols), "narrow Q6_K head");
+      check(hp::mid_takes(shape(262144, k, false, true, false), cols) == (k >= 1024), "full-range head");
+      check(!hp::mid_takes(shape(65520, k, false, true, false), cols), "fewer than 16 segments a CU");
+    }
+    check(hp::mid_takes(shape(100000, 2560, false, true, false), cols) == (cols > 2), "last round nearly empty");
+    check(hp::mid_takes(shape(131072, 2560, true, true, false), cols) == (cols > 2), "mixed types, full-range");
+    check(!hp::mid_takes(shape(131072, 1024, true, true, false), cols), "mixed types, short rows");
+    check(!hp::mid_takes(shape(131072, 2560, true, true, true), cols), "mixed types, narrow");
+    for (int k : {256, 1024, 2560, 3840})
+      for (bool q4 : {true, false}) {
+        hp::MidShape l = shape(2 * 40960, k, q4, !q4, q4);
+        l.pair = true;
+        check(hp::mid_takes(l, cols) == (cols == 4 || (cols == 3 && (!q4 || k >= 2560)) || k >= (q4 ? 3840 : 2560)), "gate/up");
+      }
+  }
+  check(!hp::mid_takes(shape(262144, 2560, false, true, false), 1), "one column");
+}
+
 }  // namespace
 
 int main() {
   grids();
+  few_columns();
   if (failures) return 1;
   std::printf("mid policy ok\n");
   return 0;

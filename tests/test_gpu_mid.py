@@ -105,6 +105,27 @@ def test_mid_geglu_bit_exact(hip, oracle, layouts, gate, up, rows, k, m):
     assert np.array_equal(_bits(got), _bits(ref))
 
 
+@pytest.mark.parametrize("kind,full,rows,k,m,launches", [
+    ("Q6_K", False, 65600, 256, 2, 1), ("Q4_K", False, 65600, 256, 4, 1),  # kquant_mfma
+    ("Q6_K", True, 65600, 1024, 2, 2), ("Q6_K", True, 65600, 1024, 4, 2),  # activation tiles, row waves
+])
+def test_two_to_four_columns_of_large_launches(hip, oracle, kind, full, rows, k, m, launches):
+    """Weights of single f16 operands stay on the one-launch matrix-core
+    kernel, full-range Q6_K weights go to the row waves."""
+    print(f"mid few columns {kind} full={full} k={k} m={m}", flush=True)
+    seed = S.derive(S.BASE_SEED, "mid-few", k, m)
+    w = _blocks(kind, seed, rows, k) if full else S.weight_blocks(kind, seed, rows, k)
+    x = S.activations(seed, m, k)
+    h = hip.createHipQuantizedWeightHandle(kind, w, k, rows)
+    try:
+        before = hip.hipResidentWeightStats()["kernelLaunches"]
+        got = hip.matMulQuantizedHipResident(h, x, k, rows, m)
+        assert hip.hipResidentWeightStats()["kernelLaunches"] - before == launches
+    finally:
+        hip.releaseHipQuantizedWeightHandle(h)
+    assert np.array_equal(_bits(got), _bits(oracle.matmul(TYPES[kind], w, x, rows, threads=8)))
+
+
 def test_capture_without_scratch(hip, oracle):
     """A captured call of eight columns on a stream that no call has sized
     scratch for is accepted (its kernels without activation tiles run), with
