@@ -545,7 +545,8 @@ int32_t run_matvec(size_t count, Handle *const *hs, const float *d_input, size_t
   State &s = st();
   if (cols == 0) return HP_OK;
   if (tail_in && !tail_in->part) tail_in = nullptr;
-  const MfmaFit fit = mfma_fit(count, hs);
+  MfmaFit fit = mfma_fit(count, hs);
+  fit.folded = s.prefill_folds && (norm || tiles_in);
   int kind = prefill_kind(cols, fit);
   uint8_t *pre = nullptr;  // the prefill kernels' scratch
   if (kind == 3) {

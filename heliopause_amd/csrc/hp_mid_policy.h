@@ -16,6 +16,7 @@ struct MidShape {
   bool q4, q6;     // some weight is Q4_K, Q6_K
   bool f16;        // every weight is exact in single f16 operands (no full-range Q6_K scales)
   bool pair;       // gate and up with their GeGLU
+  bool folded;     // the launch before writes the activation tiles
   int cus;
 };
 
@@ -69,8 +70,29 @@ inline bool mid_takes_few(const MidShape &l, size_t cols) {
   return l.nb >= 4 && (cols > 2 || mid_rounds_full(l));
 }
 
+// Five to eight columns for which kquant_mfma's one launch (single-operand
+// weights) is faster than a launch that writes activation tiles and this
+// kernel: short rows.  Times are this kernel's over that one's.
+inline bool mfma_takes(const MidShape &l, size_t cols) {
+  if (!l.f16 || l.pair || l.folded || cols > 8) return false;
+  if (l.q4 && l.q6 && l.segs >= 2ll * l.cus) {
+    // class pairs for want of one type: 8192 rows of 1 and 2 blocks 1.20,
+    // 1.07, of 3 blocks 0.98; 16384 of 3 blocks 1.05 to 1.21, of 4 0.98;
+    // 32768 to 131072 of 4 to 6 blocks 1.05 to 1.32, of 10 blocks 0.97
+    return l.nb <= (l.segs >= 8ll * l.cus ? 6 : l.segs >= 4ll * l.cus ? 3 : 2);
+  }
+  // many rows: Q4_K 32768 of one block 0.95, 65536 0.78; Q6_K 32768 1.05, 65536 0.86
+  if (l.segs >= (l.q4 ? 8ll : 16ll) * l.cus) return false;
+  // one block 1.02 to 1.16
+  if (l.nb == 1) return true;
+  // row waves of Q6_K: two blocks 1.05 to 1.14, three 1.05 to 1.11 at five
+  // columns and 0.92 to 0.95 at six to eight; four 0.9 and less
+  return l.q6 && mid_row_waves(l) && (l.nb == 2 || (l.nb == 3 && cols == 5));
+}
+
 inline bool mid_takes(const MidShape &l, size_t cols) {
-  return mid_grid_fits(l, cols) && (cols >= kMidMinCols || mid_takes_few(l, cols));
+  if (!mid_grid_fits(l, cols)) return false;
+  return cols >= kMidMinCols ? !mfma_takes(l, cols) : mid_takes_few(l, cols);
 }
 
 }  // namespace hp

@@ -66,11 +66,36 @@ void few_columns() {
   check(!hp::mid_takes(shape(262144, 2560, false, true, false), 1), "one column");
 }
 
+// Five to eight columns of short rows in single f16 operands: kquant_mfma,
+// unless the activation tiles come without a launch of their own.
+void short_rows() {
+  for (size_t cols = 5; cols <= 9; cols++) {
+    const bool to8 = cols <= 8;
+    for (long long rows : {1, 16, 2560, 10240, 32752}) {
+      hp::MidShape l = shape(rows, 256, true, false, true);
+      check(hp::mid_takes(l, cols) == !to8, "one block");
+      l.folded = true;
+      check(hp::mid_takes(l, cols), "one block, folded");
+      check(hp::mid_takes(shape(rows, 256, false, true, false), cols), "one block, full-range");
+      check(hp::mid_takes(shape(rows, 2560, true, true, true), cols), "ten blocks");
+    }
+    check(hp::mid_takes(shape(32768, 256, true, false, true), cols), "one block, many rows");
+    check(hp::mid_takes(shape(32768, 256, false, true, true), cols) == !to8, "one block, many rows of Q6_K");
+    check(hp::mid_takes(shape(8192, 512, false, true, true), cols) == !to8, "Q6_K row waves, two blocks");
+    check(hp::mid_takes(shape(8192, 768, false, true, true), cols) == (cols != 5), "Q6_K row waves, three blocks");
+    check(hp::mid_takes(shape(8160, 512, false, true, true), cols), "Q6_K class pairs, two blocks");
+    check(hp::mid_takes(shape(8192, 512, true, false, true), cols), "Q4_K row waves, two blocks");
+    check(hp::mid_takes(shape(65536, 1536, true, true, true), cols) == !to8, "mixed, six blocks");
+    check(hp::mid_takes(shape(16384, 1024, true, true, true), cols), "mixed, four blocks");
+  }
+}
+
 }  // namespace
 
 int main() {
   grids();
   few_columns();
+  short_rows();
   if (failures) return 1;
   std::printf("mid policy ok\n");
   return 0;

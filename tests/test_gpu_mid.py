@@ -127,6 +127,30 @@ def test_two_to_four_columns_of_large_launches(hip, oracle, kind, full, rows, k,
     assert np.array_equal(_bits(got), _bits(oracle.matmul(TYPES[kind], w, x, rows, threads=8)))
 
 
+@pytest.mark.parametrize("specs,k,m,launches", [
+    ([("Q4_K", 2560)], 256, 8, 1), ([("Q6_K", 300), ("Q4_K", 100)], 256, 5, 1), ([("Q6_K", 8200)], 512, 6, 1),
+    ([("Q6_K", 8200)], 768, 5, 1), ([("Q6_K", 8200)], 768, 6, 2), ([("Q4_K", 2560)], 256, 9, 2),
+])
+def test_short_rows_of_five_to_eight_columns(hip, oracle, specs, k, m, launches):
+    """Short rows in single f16 operands: kquant_mfma's one launch, or the
+    activation tiles and the mid kernel."""
+    print(f"mid short rows {specs} k={k} m={m}", flush=True)
+    seed = S.derive(S.BASE_SEED, "mid-short", k, m)
+    ws = [S.weight_blocks(t, S.derive(seed, i), r, k) for i, (t, r) in enumerate(specs)]
+    x = S.activations(seed, m, k)
+    hs = [hip.createHipQuantizedWeightHandle(t, w, k, r) for (t, r), w in zip(specs, ws)]
+    try:
+        before = hip.hipResidentWeightStats()["kernelLaunches"]
+        got = hip.matMulQuantizedHipResidentMulti(hs, x, k, m) if len(hs) > 1 else [
+            hip.matMulQuantizedHipResident(hs[0], x, k, specs[0][1], m)]
+        assert hip.hipResidentWeightStats()["kernelLaunches"] - before == launches
+    finally:
+        for h in hs:
+            hip.releaseHipQuantizedWeightHandle(h)
+    for (t, r), w, g in zip(specs, ws, got):
+        assert np.array_equal(_bits(g), _bits(oracle.matmul(TYPES[t], w, x, r, threads=8)))
+
+
 def test_capture_without_scratch(hip, oracle):
     """A captured call of eight columns on a stream that no call has sized
     scratch for is accepted (its kernels without activation tiles run), with
