@@ -379,8 +379,8 @@ int chunk_kind(size_t cols, MfmaFit fit) {
 int prefill_kind(size_t cols, MfmaFit fit) {
   const State &s = st();
   const int kind = chunk_kind(cols, fit);
-  if (s.matvec_kernel == 0 && kind != 2 && fit.tiles && cols <= kMaxTileCols && mid_lds_bytes() <= s.max_lds &&
-      mid_takes(fit, cols))
+  if (s.matvec_kernel == 0 && kind != 2 && !(kind == 1 && prefill_takes(fit, cols)) && fit.tiles &&
+      cols <= kMaxTileCols && mid_lds_bytes() <= s.max_lds && mid_takes(fit, cols))
     return 3;
   return kind;
 }

@@ -90,6 +90,28 @@ inline bool mfma_takes(const MidShape &l, size_t cols) {
   return l.q6 && mid_row_waves(l) && (l.nb == 2 || (l.nb == 3 && cols == 5));
 }
 
+// Hundreds of columns (host-pointer calls, which keep to bit-exact kernels) of
+// class-pair launches in single f16 operands, for which the bit-exact prefill
+// kernel with its 64-column tiles is faster: a class pair reads a column's
+// activation tiles once per 16-row segment, and over short rows the exchange
+// of the chains costs as much as the blocks.  Times are this kernel's over that
+// one's, measured at 16 to 500 segments.
+inline bool prefill_takes(const MidShape &l, size_t cols) {
+  if (!l.f16 || mid_row_waves(l)) return false;  // row waves 0.41 to 0.74
+  const long long work = l.segs * (long long)cols;
+  // one block 0.92 to 1.01 up to 65536 segment columns, 1.08 to 1.71 from
+  // 81920; 16 segments 1.08 at 1536 columns, 1.25 at 2048
+  if (l.nb == 1) return work >= 80000 || cols >= 2048;
+  // two blocks 0.97 to 1.0 at 81920, 1.04 to 1.34 from 122880
+  if (l.nb == 2) return work >= 120000;
+  // four blocks 0.77 to 0.95.  Long rows, whose activation tiles pass the L2
+  // (128 segments and more): 15 to 40 blocks 0.81 to 1.02 at 768 columns, 1.05
+  // to 1.21 at 1024; 10 blocks 0.96 to 0.99 at 1024, 0.97 to 1.09 from 1536;
+  // 16 segments 0.5 to 1.1; gate/up 0.5 to 0.95
+  if (l.pair || l.segs < 128) return false;
+  return cols >= 1536 ? l.nb >= 10 : cols >= 1024 && l.nb >= 15;
+}
+
 inline bool mid_takes(const MidShape &l, size_t cols) {
   if (!mid_grid_fits(l, cols)) return false;
   return cols >= kMidMinCols ? !mfma_takes(l, cols) : mid_takes_few(l, cols);

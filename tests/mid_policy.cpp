@@ -90,12 +90,31 @@ void short_rows() {
   }
 }
 
+// Many columns of host calls: the bit-exact prefill kernel for short rows of
+// enough work and for long rows of class pairs, never below 64 columns.
+void many_columns() {
+  for (int nb = 1; nb <= 40; nb++)
+    for (long long rows : {16, 2560, 8176})
+      for (size_t cols = 1; cols < 64; cols++) check(!hp::prefill_takes(shape(rows, 256 * nb, true, false, true), cols), "below 64");
+  check(!hp::prefill_takes(shape(2560, 256, true, false, true), 256), "one block, 40960");
+  check(hp::prefill_takes(shape(2560, 256, true, false, true), 512), "one block, 81920");
+  check(!hp::prefill_takes(shape(2560, 512, false, true, true), 512), "two blocks, 81920");
+  check(hp::prefill_takes(shape(2560, 512, false, true, true), 768), "two blocks, 122880");
+  check(!hp::prefill_takes(shape(5120, 1024, true, false, true), 4096), "four blocks");
+  check(hp::prefill_takes(shape(2560, 10240, false, true, true), 1024), "40 blocks");
+  check(!hp::prefill_takes(shape(2560, 10240, false, true, true), 1023), "40 blocks, fewer columns");
+  check(hp::prefill_takes(shape(3072, 2560, true, true, true), 1536), "10 blocks, mixed");
+  check(!hp::prefill_takes(shape(2560, 10240, false, true, false), 4096), "full-range");
+  check(!hp::prefill_takes(shape(8192, 10240, false, true, true), 4096), "row waves");
+}
+
 }  // namespace
 
 int main() {
   grids();
   few_columns();
   short_rows();
+  many_columns();
   if (failures) return 1;
   std::printf("mid policy ok\n");
   return 0;

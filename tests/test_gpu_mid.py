@@ -151,6 +151,28 @@ def test_short_rows_of_five_to_eight_columns(hip, oracle, specs, k, m, launches)
         assert np.array_equal(_bits(g), _bits(oracle.matmul(TYPES[t], w, x, r, threads=8)))
 
 
+@pytest.mark.parametrize("specs,k,m", [
+    ([("Q4_K", 2560)], 256, 520), ([("Q6_K", 2000), ("Q4_K", 600)], 2560, 1540), ([("Q6_K", 2100)], 3840, 1030),
+])
+def test_many_columns_of_host_calls(hip, oracle, layouts, specs, k, m):
+    """Host calls of the sizes that the bit-exact prefill kernel takes."""
+    print(f"mid many columns {specs} k={k} m={m} both={layouts}", flush=True)
+    seed = S.derive(S.BASE_SEED, "mid-many", k, m)
+    ws = [S.weight_blocks(t, S.derive(seed, i), r, k) for i, (t, r) in enumerate(specs)]
+    part = S.activations(seed, 40, k)
+    x = np.resize(part, (m, k))  # column c is part[c % 40]
+    hs = [hip.createHipQuantizedWeightHandle(t, w, k, r) for (t, r), w in zip(specs, ws)]
+    try:
+        got = hip.matMulQuantizedHipResidentMulti(hs, x, k, m) if len(hs) > 1 else [
+            hip.matMulQuantizedHipResident(hs[0], x, k, specs[0][1], m)]
+    finally:
+        for h in hs:
+            hip.releaseHipQuantizedWeightHandle(h)
+    for (t, r), w, g in zip(specs, ws, got):
+        ref = oracle.matmul(TYPES[t], w, part, r, threads=8).reshape(40, r)
+        assert np.array_equal(_bits(g), _bits(np.resize(ref, (m, r))))
+
+
 def test_capture_without_scratch(hip, oracle):
     """A captured call of eight columns on a stream that no call has sized
     scratch for is accepted (its kernels without activation tiles run), with
