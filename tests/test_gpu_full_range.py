@@ -3,9 +3,13 @@ them) on the matrix cores, where sc * (q - 32) needs two exact f16 operands.
 
 An operand rounded to one f16 would be off by one unit in up to 4096, about
 1e-5 of an output, so the fast prefill kernel is compared against f64 sums of
-the exact integers with the rounding bound of its f32 tail: per block three
+the exact integers with the rounding bound of its f32 sums: per block three
 roundings (dw * D, times dx, the running sum; each at most 2^-24 of the terms
-so far), block ranges add one more each, so (3 nb + 8) 2^-24 sum_b |t_b|.
+so far), block ranges add one more each, so (3 nb + 8) 2^-24 sum_b |t_b|.  D
+itself, a block's integer sum, is exact while its partial sums stay within
+2^24; a block whose products add up to more (|p| summed, up to 2^27) rounds
+at most once per four products of either operand, 128 times, each by 2^-24 of
+that sum.
 """
 import ctypes
 
@@ -37,6 +41,22 @@ def _terms(oracle, w, x, rows):
     xq = (qs.astype(np.float64).reshape(m, -1, 256) * d.astype(np.float64)[:, :, None])
     deq = np.stack([oracle.dequantize(3, w[r], k) for r in range(rows)]).astype(np.float64).reshape(rows, -1, 256)
     return np.einsum("rbe,mbe->rmb", deq, xq)
+
+
+def _bound(oracle, w, x, rows):
+    """(f64 sums, rounding bounds), [rows][m], of the module's first lines."""
+    m, k = x.shape
+    qs, d, _ = oracle.quantize_q8_k(x)
+    xq = np.abs(qs.astype(np.float64)).reshape(m, -1, 256)
+    b = w.reshape(rows, -1, 210)
+    dw = b[:, :, 208:210].copy().view(np.float16).astype(np.float64)[:, :, 0]
+    deq = np.stack([oracle.dequantize(3, w[r], k) for r in range(rows)]).astype(np.float64).reshape(rows, -1, 256)
+    ints = np.abs(np.divide(deq, dw[:, :, None], out=np.zeros_like(deq), where=dw[:, :, None] != 0))  # |sc (q - 32)|
+    p = np.matmul(ints.transpose(1, 0, 2), xq.transpose(1, 2, 0))  # [nb][rows][m], sums of |products|
+    unit = np.abs(dw).T[:, :, None] * np.abs(d.astype(np.float64)).reshape(m, -1).T[:, None, :]
+    t = _terms(oracle, w, x, rows)
+    rounded = np.where(p > 2.0 ** 24 * (1 - 1e-9), p * unit, 0.0).sum(0)
+    return t.sum(2), ((3 * (k // 256) + 8) * np.abs(t).sum(2) + 128 * rounded) * 2.0 ** -24
 
 
 def _device(a):
@@ -77,11 +97,10 @@ def test_fast_prefill_full_range(hip, oracle, layouts, rows, k, m):
     finally:
         hip.releaseHipQuantizedWeightHandle(h6)
         hip.releaseHipQuantizedWeightHandle(h4)
-    t = _terms(oracle, w6, x, rows)
-    bound = (3 * (k // 256) + 8) * 2.0 ** -24 * np.abs(t).sum(2)
+    want, bound = _bound(oracle, w6, x, rows)
     for got in (alone, joined):
         g = got.cpu().numpy().reshape(m, rows).T.astype(np.float64)
-        assert np.all(np.abs(g - t.sum(2)) <= bound), np.max(np.abs(g - t.sum(2)) / np.maximum(bound, 1e-300))
+        assert np.all(np.abs(g - want) <= bound), np.max(np.abs(g - want) / np.maximum(bound, 1e-300))
     ref4 = oracle.matmul(1, w4, x, 48, threads=8)
     for got in (q4, q4_alone):
         g = got.cpu().numpy()
@@ -120,8 +139,7 @@ def test_full_range_capture_without_scratch(hip, oracle):
     seed = S.derive(S.BASE_SEED, "full-range-capture")
     w, x = _full_range(seed, rows, k), S.activations(seed, m, k)
     ref = oracle.matmul(3, w, x, rows)
-    t = _terms(oracle, w, x, rows)
-    bound = (3 * (k // 256) + 8) * 2.0 ** -24 * np.abs(t).sum(2)
+    want, bound = _bound(oracle, w, x, rows)
     h = hip.createHipQuantizedWeightHandle("Q6_K", w, k, rows)
     stream = torch.cuda.Stream()
     print("full range capture", flush=True)
@@ -144,7 +162,7 @@ def test_full_range_capture_without_scratch(hip, oracle):
                 torch.cuda.synchronize()
                 got = out.cpu().numpy()
                 if sized:
-                    assert np.all(np.abs(got.reshape(m, rows).T.astype(np.float64) - t.sum(2)) <= bound)
+                    assert np.all(np.abs(got.reshape(m, rows).T.astype(np.float64) - want) <= bound)
                 else:
                     assert np.array_equal(got.view(np.uint32), ref.reshape(-1).view(np.uint32))
             del graph

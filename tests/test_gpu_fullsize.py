@@ -338,19 +338,21 @@ def test_decode_step_42_layers_with_head(hip, oracle, head_blocks, tokens):
             _topk_near_ties(g_ids, got_logits[r], end_logits[r].astype(np.float64), 40, f"draft row {r}")
 
 
-@pytest.mark.parametrize("tokens", [2, 3, 4, 5, 6, 7, 8])
-def test_draft_input_images_bit_identical(hip, tokens):
+@pytest.mark.parametrize("tokens,kernel", [(2, 0), (3, 0), (4, 0), (2, 1), (5, 1), (6, 1), (7, 1), (8, 1)])
+def test_draft_input_images_bit_identical(hip, tokens, kernel):
     """The pre-quantised inputs of a draft step (the Q/K/V input written by the
     norm launch, the down input written by the GeGLU launch) against every
     projection quantising its own f32 input: the same layer at full size run
-    both ways gives identical residual streams and caches."""
+    both ways gives identical residual streams and caches.  The vector-ALU
+    kernels read these images: at two to four tokens on the automatic policy
+    (kernel 0), from five on where they are selected (kernel 1)."""
     import torch
 
     shape = DM.ModelShape()
     data = DM.layer_host_data(shape, S.derive(S.BASE_SEED, "images", tokens), 0)
     x = S.activations(S.derive(S.BASE_SEED, "images-x", tokens), tokens, shape.hidden) * 4
     results = []
-    print(f"draft images tokens={tokens}", flush=True)
+    print(f"draft images tokens={tokens} kernel={kernel}", flush=True)
     for images in (True, False):
         model = DM.HipDecodeModel(shape)
         model.add_layer(data)
@@ -358,11 +360,13 @@ def test_draft_input_images_bit_identical(hip, tokens):
         dpos = _dev(np.array([shape.capacity - tokens], np.int32))
         try:
             hip.setInputImages(images)
+            hip.setMatvecKernel(kernel)
             model.run_layers(dx.data_ptr(), dpos.data_ptr(), tokens=tokens)
             torch.cuda.synchronize()
             results.append((dx.cpu().numpy(), model.caches[0][0].cpu().numpy(), model.caches[0][1].cpu().numpy()))
         finally:
             hip.setInputImages(True)
+            hip.setMatvecKernel(0)
             model.release()
     (h1, k1, v1), (h2, k2, v2) = results
     assert np.array_equal(_bits(h1), _bits(h2)), _first_diff(h1, h2)

@@ -160,10 +160,12 @@ def _q6k_full_range_scales(seed, rows, k):
 @pytest.mark.parametrize("kernel_id", [0, 1, 2, 3, 4, 5, 6, 7, 8],
                          ids=["auto", "valu", "mfma", "half", "prefill", "fast", "wide", "wide-whole", "wide-half"])
 def test_q6k_full_range_scales(hip, oracle, kernel_id):
-    """Q6_K scales beyond +-66 make sc * (q - 32) inexact as an f16 matrix-core
-    operand; such weights run the vector-ALU kernels under every selector, so
-    the results stay bit-exact (alone and in a launch with Q4_K weights) at
-    decode and prefill column counts."""
+    """Q6_K scales beyond +-66 make sc * (q - 32) inexact as one f16 matrix-core
+    operand; such weights run the vector-ALU kernels under every forced
+    selector and, as two exact operands, the mid kernels under the automatic
+    one from five columns of a host call on, so the results stay bit-exact
+    (alone and in a launch with Q4_K weights) at decode and prefill column
+    counts."""
     k = 2560
     seed = S.derive(S.BASE_SEED, "q6kfull", kernel_id)
     w6 = _q6k_full_range_scales(seed, 300, k)

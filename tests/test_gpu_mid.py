@@ -49,7 +49,9 @@ def _bits(a):
     ([("Q6_K", 8500)], 256, 16),                        # one block per item
     ([("Q6_K", 20000)], 768, 30),                       # several items per workgroup, 3 blocks
     ([("Q4_K", 9000), ("Q4_K", 8200)], 1280, 50),       # two weights; 2 column groups of 32
-    ([("Q6_K", 66000)], 256, 2),                        # large launches from two columns
+    ([("Q6_K", 66000)], 256, 2),                        # two columns of one block: vector ALU
+    ([("Q4_K", 40)], 10240, 5), ([("Q6_K", 33)], 10240, 16),   # long rows: single classes, 16 columns
+    ([("Q4_K", 24), ("Q6_K", 40)], 10240, 17), ([("Q6_K", 50)], 10240, 32), ([("Q4_K", 17)], 5120, 31),  # and 32
 ])
 def test_mid_bit_exact(hip, oracle, layouts, specs, k, m):
     """Device and host calls."""
@@ -82,6 +84,7 @@ def test_mid_bit_exact(hip, oracle, layouts, specs, k, m):
 @pytest.mark.parametrize("gate,up,rows,k,m", [
     ("Q4_K", "Q4_K", 200, 768, 21), ("Q4_K", "Q6_K", 48, 1280, 40), ("Q6_K", "Q6_K", 4200, 256, 5),
     ("Q4_K", "Q4_K", 4112, 512, 40), ("Q4_K", "Q4_K", 17000, 256, 11),
+    ("Q4_K", "Q4_K", 4080, 512, 33), ("Q6_K", "Q6_K", 2050, 768, 63), ("Q6_K", "Q4_K", 2049, 512, 50),  # pairs of 32
 ])
 def test_mid_geglu_bit_exact(hip, oracle, layouts, gate, up, rows, k, m):
     import torch
@@ -203,6 +206,46 @@ def test_capture_without_scratch(hip, oracle):
                 torch.cuda.synchronize()
                 assert np.array_equal(_bits(out.cpu().numpy()), _bits(ref)), sized
             del graph
+    finally:
+        hip.releaseHipQuantizedWeightHandle(h)
+        hip.lib().hp_hip_release_stream_scratch(ctypes.c_void_p(stream.cuda_stream))
+
+
+def test_capture_of_40_columns_needs_scratch(hip, oracle):
+    """From 32 columns of single-operand weights on, every kernel of the
+    automatic choice needs scratch: a capture on a stream without is refused,
+    one after an uncaptured call of the shape is not."""
+    import torch
+
+    rows, k, m = 64, 768, 40
+    w, x = _blocks("Q4_K", 5, rows, k), S.activations(6, m, k)
+    h = hip.createHipQuantizedWeightHandle("Q4_K", w, k, rows)
+    stream = torch.cuda.Stream()
+    try:
+        dx, out = torch.from_numpy(x.reshape(-1)).to("cuda:0"), torch.empty(rows * m, device="cuda:0")
+        torch.cuda.synchronize()
+        run = lambda: hip.matmul_multi_device([h.handle], dx.data_ptr(), k, m, [out.data_ptr()],  # noqa: E731
+                                              [out.numel()], stream.cuda_stream)
+        refused, graph = None, torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            out.zero_()
+            try:
+                run()
+            except RuntimeError as e:
+                refused = str(e)
+        assert refused and "before graph capture" in refused
+        run()
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            run()
+        for _ in range(2):
+            out.zero_()
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert np.array_equal(_bits(out.cpu().numpy()), _bits(oracle.matmul(1, w, x, rows)))
+        del graph
     finally:
         hip.releaseHipQuantizedWeightHandle(h)
         hip.lib().hp_hip_release_stream_scratch(ctypes.c_void_p(stream.cuda_stream))

@@ -323,14 +323,16 @@ def test_prefill_chunks_through_layers(hip, D, kernel):
     _check_rows(got_out, ref_out, "chunked output norm", tol)
 
 
-@pytest.mark.parametrize("tokens", [512, 100])
+@pytest.mark.parametrize("tokens", [512, 100, 40, 21, 9, 5])
 def test_prefill_folds_bit_identical(hip, tokens):
     """The launch folds of a prefill chunk (activation tiles written by the
     norm launches and by the attention's slice merge, block-range sums added
     by the next launch, f16 queries from the attention prologue) against the
     plain launches (hp_hip_set_prefill_folds(0)): two layers of the model's
-    shape at 512 and 100 tokens (the last 64-column tile padded), hidden
-    states, output norm and both layers' caches bit-identical."""
+    shape at 512 and 100 tokens (the last 64-column tile padded), and at 40,
+    21, 9 and 5, whose projections take 16-column tiles (padded to 64, 32, 16
+    and 16 columns; at 5 from the norm launches only): hidden states, output
+    norm and both layers' caches bit-identical."""
     import torch
 
     shape = DM.ModelShape()

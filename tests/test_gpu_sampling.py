@@ -83,6 +83,38 @@ def test_sample_device_matches_oracle(opts, k, count):
     assert int(state.cpu().numpy().view(np.uint32)[0]) == ref_rng.state
 
 
+@pytest.mark.parametrize("opts", [OPTION_SETS[1], OPTION_SETS[7]], ids=["sampled", "greedy"])
+@pytest.mark.parametrize("cols", [1, 16, 17, 40])
+def test_sample_columns_past_the_waves(opts, cols):
+    """A wave per column, 16 waves: one column, as many as waves, and second
+    and third trips of a wave; the generator state after two calls."""
+    import torch
+
+    k = 40
+    ids, vals = _columns(np.random.default_rng(cols), cols, k, k, 3.0)
+    dev = torch.device("cuda:0")
+    d_ids, d_vals = torch.from_numpy(ids.view(np.int32)).to(dev), torch.from_numpy(vals).to(dev)
+    state = torch.from_numpy(np.array([99], np.uint32).view(np.int32)).to(dev)
+    tokens, kept = (torch.zeros(cols, dtype=torch.int32, device=dev) for _ in range(2))
+    probs = torch.zeros(cols * k, dtype=torch.float64, device=dev)
+    print(f"sample cols={cols} opts={opts}", flush=True)
+    ref_rng = SM.DeterministicRng(99)
+    for call in range(2):
+        H.sample_device(d_ids.data_ptr(), d_vals.data_ptr(), cols, k, k, opts, state.data_ptr(), tokens.data_ptr(),
+                        probs.data_ptr(), kept.data_ptr())
+        torch.cuda.synchronize()
+        got_tokens, got_kept = tokens.cpu().numpy(), kept.cpu().numpy()
+        got_probs = probs.cpu().numpy().reshape(cols, k)
+        for c in range(cols):
+            cands = [{"id": int(ids[c, j]), "value": float(vals[c, j])} for j in range(k)]
+            dist = SM.token_sampling_distribution(cands, opts)
+            assert got_tokens[c] == SM.sample_next_token(cands, opts, ref_rng), (call, c)
+            assert got_kept[c] == len(dist), (call, c)
+            want = np.array([d["probability"] for d in dist], np.float64)
+            assert np.array_equal(got_probs[c, :len(dist)].view(np.uint64), want.view(np.uint64)), (call, c)
+        assert int(state.cpu().numpy().view(np.uint32)[0]) == ref_rng.state, call
+
+
 @pytest.mark.parametrize("m,softcap", [(1, 0.0), (4, 30.0)])
 def test_head_topk_sample_matches_oracle(hip, oracle, m, softcap):
     """forwardOutput + sampleNextToken per column in one call."""
