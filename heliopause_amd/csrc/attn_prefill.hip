@@ -40,7 +40,7 @@
 // values transposed (V^T, dim rows of 32 keys) -- so the next tile is
 // stored while this one is read and one barrier per tile suffices.  Row
 // strides are padded so the 16 lanes of an MFMA operand read hit distinct
-// 16-byte slots, and the staging stores are laid out to do the same.
+// 16-byte slots, and the staging stores are laid out so that theirs do.
 //
 // Every token block of one (KV head, slice) reads the same keys and values.
 // Workgroup i runs on XCD i % 8, so the work items are dealt out such that
@@ -223,8 +223,8 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const AttnArgs a, 
   // of one row: with a row per lane the L1's address unit was busy half the
   // kernel's time).  Keys: a quarter row of key k_j,
   // 16-byte chunks k_e + 8 i, turned by 7 chunks on odd rows.  With the
-  // padded strides each store's 8 (and 16) consecutive lanes then fill
-  // distinct 16-byte slots of 128 (and 256) bytes.
+  // padded strides each store's 16 consecutive lanes then fill the 16
+  // distinct 16-byte slots of 256 bytes (all 64 banks).
   const int v_q = (tid >> 2) & 3, v_dg = (tid & 3) | ((tid >> 4) << 2);  // columns 8 v_q.., dims 4 v_dg..
   const int k_j = tid >> 3, k_e = tid & 7;    // key k_j, chunks (k_e + 8 i + 7 (k_j & 1)) % 32
   const int k_rot = k_e + 7 * (k_j & 1);

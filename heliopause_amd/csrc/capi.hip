@@ -322,19 +322,20 @@ int cols_per_launch(const TileGeom &g, size_t max_lds) {
   return 0;
 }
 
-// Kernel choice.  The matrix-core kernel's cost barely grows with the column
-// count but each wave walks its 16-row tile block by block, so it needs many
-// tiles to hide memory latency; the vector-ALU kernel's cost grows with the
-// columns (and it spills registers beyond four).  Measured on MI355X: the
-// matrix cores win from five columns on, and from two columns on when the
-// launch has >= 1024 tiles (16 rows each); one column stays on the vector
-// ALU.  Both need their LDS (the columns' Q8_K for every block) to fit.
-// Prefill kernels (matrix cores, columns in tiles of 64, weights read once per
-// column tile) for many columns.  From kFastMinCols columns the automatic
-// policy takes the fast one, whose outputs agree with the reference within the
-// 1e-4 relative tolerance of projections (M >= 64 prefill chunks); selector 4
-// forces the bit-exact one, 5 the fast one.  Below kPrefillMinCols the decode
-// kernels, which read the weights once per 8 columns, are as fast.
+// Kernel choice, by column count: the vector-ALU kernels (use_half, use_wide
+// and the plain one) for one column and most launches of two to four; the mid
+// kernels (kquant_mid.hip) from five columns, or two of some large launches
+// (hp_mid_policy.h); the fast prefill kernel from kFastMinCols columns of
+// device calls.  The decode matrix-core kernel (use_mfma, eight columns a
+// launch) keeps large launches of two to four columns and short rows of five
+// to eight; the bit-exact prefill kernel (64-column tiles, weights read once
+// per tile) some host calls of hundreds of columns.  Where the mid kernels
+// have no scratch (try_scratch) or do not fit, a launch runs as if they were
+// not there: decode kernels below kPrefillMinCols columns, the bit-exact
+// prefill kernel from there.  Outputs of the fast kernel agree with the
+// reference within the 1e-4 relative tolerance of projections; every other
+// kernel gives its bits.  Selector 4 forces the bit-exact prefill kernel, 5
+// the fast one.
 constexpr size_t kPrefillMinCols = 32;
 constexpr size_t kFastMinCols = 64;
 constexpr size_t kMaxTileCols = 65535;  // columns of one launch of the prefill and mid kernels
@@ -374,8 +375,9 @@ int chunk_kind(size_t cols, MfmaFit fit) {
 // the matrix cores, bit-exact) for the launches of hp_mid_policy.h below the
 // fast kernel's column counts, and at every count of the host-pointer calls.
 // A launch whose activation tiles cannot be had (a captured call that no
-// earlier call has sized scratch for, which the kernels of chunk_kind 0 do not
-// need) runs as chunk_kind says: the same bits.
+// earlier call has sized scratch for, or no memory) runs as chunk_kind says:
+// the same bits, and no scratch where that is 0 (below 32 columns, or
+// full-range Q6_K).
 int prefill_kind(size_t cols, MfmaFit fit) {
   const State &s = st();
   const int kind = chunk_kind(cols, fit);
@@ -2527,7 +2529,8 @@ int32_t hp_hip_decode_layers_device(const hp_hip_decode_layer_t *layers, size_t 
   const size_t M = chunk;  // rows of every scratch buffer
   // scratch ([M] rows each): xn, q, k, v, q after RoPE, attention, o, x1, h, y;
   // attention partials; RoPE tables [M][128] cos, sin
-  // (2..8 tokens) the Q/K/V and down inputs as pre-quantised images
+  // (2..8 tokens, where the projections run the vector-ALU kernels: up to
+  // four, or as selected) the Q/K/V and down inputs as pre-quantised images
   auto al = [](size_t n) { return (n + 63) & ~(size_t)63; };
   const bool images = M >= 2 && M <= (size_t)kMaxTokens;
   const size_t img_x = images ? q8_image_bytes((int)M, (int)(hidden / kQK)) / sizeof(float) : 0;

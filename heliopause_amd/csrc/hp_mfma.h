@@ -82,7 +82,10 @@ __device__ __forceinline__ half8 cat(half2v a, half2v b, half2v c, half2v d) {
 // (sc & ~1) * (q - 32) (even) and (sc & 1) * (q - 32), each its own MFMA on
 // the same accumulator.  Every partial sum over one class stays an integer of
 // at most 2^24: 32 x 32 x 128 x 128, and the odd parts only shrink the terms
-// of negative odd scales (127 = 128 - 1) and complete the positive ones.
+// of negative odd scales (127 = 128 - 1) and complete the positive ones.  The
+// mid kernels start an accumulator per class, so theirs are exact; the fast
+// prefill kernel carries one over a block's eight classes (up to 2^27), which
+// rounds as its other f32 sums do where a partial sum passes 2^24.
 // Scales of a 4-byte group word as even parts (s0, s1), (s2, s3) and odd masks.
 __device__ __forceinline__ void q6_split_scales(half2v (&S)[2], uint32_t (&M)[2], uint32_t gs) {
   const uint32_t u = gs ^ 0x80808080u;  // s + 128 (128 is even: same parity)

@@ -20,10 +20,15 @@ struct MidShape {
   int cus;
 };
 
-// From five columns on (measured against the vector-ALU and kquant_mfma
-// kernels: five columns of Q/K/V 14.3 -> 9.5 us, of the FFN 61.8 -> 36.0; at
-// four O 6.9 -> 9.1, Q/K/V 9.8 -> 9.8, with the launch that writes the
-// activation tiles), and from two on for some launches of 16 segments a CU.
+// From five columns on: against the vector-ALU kernels (full-range Q6_K) and
+// kquant_mfma, five columns of Q/K/V 15.5 -> 10.4 us, O 17.4 -> 9.7, down 35.0
+// -> 18.9, the FFN 64.1 -> 38.3.  Fewer columns stay on the kernels whose
+// launches quantise their own input: at three Q/K/V 9.5 against 10.4 us here,
+// O 7.5 against 9.7, down 17.3 against 19.0, the FFN 35.9 against 37.3; at two
+// 8.3, 6.3, 13.1 and 28.3 against 10.5, 9.6, 18.9 and 37.2.  At four the line
+// is not where each launch would have it: O 8.1 against 9.7, but Q/K/V 11.3
+// against 10.4, down 21.2 against 18.9, the FFN 42.9 against 37.9.  From two
+// columns on for some launches of 16 segments a CU.
 constexpr size_t kMidMinCols = 5;
 constexpr int kMidLargeSegs = 16;  // 16-row segments per CU
 

@@ -1,7 +1,7 @@
-// kquant_mid.hip -- Q4_K / Q6_K x Q8_K projections of 2 to 63 columns (a
-// draft, a short prompt; host calls of any count) on the gfx950 matrix cores,
-// bit-exact with the reference's WASM path (packages/engine/wasm-kernels/
-// src/lib.rs:224-426 with the vec-dots 2116-2172 and 1923-1968).
+// kquant_mid.hip -- Q4_K / Q6_K x Q8_K projections of 5 to 63 columns (a
+// draft, a short prompt; some of 2 to 4; host calls of more) on the gfx950
+// matrix cores, bit-exact with the reference's WASM path (packages/engine/
+// wasm-kernels/src/lib.rs:224-426 with the vec-dots 2116-2172 and 1923-1968).
 //
 // Numerics are those of kquant_prefill.hip's bit-exact kernel: per (row,
 // column, block) one v_mfma_f32_16x16x32_f16 per lane class l gives aux32[l]
@@ -20,9 +20,10 @@
 //
 // Measured on MI355X against what these launches ran before (the vector-ALU
 // kernels 8 columns at a time, or kquant_mfma's 8): with full-range Q6_K
-// weights, three layers of 21 tokens 1099 -> 323 us, of 5 tokens 353 -> 257;
-// gate/up + GeGLU + down 62 -> 36 us at 5 columns, 223 -> 53 at 21, 480 -> 79
-// at 60; the 262144-row head at 5 columns 416 -> 137 us.
+// weights, three layers of 21 tokens 1086 -> 271 us, of 5 tokens 345 -> 245;
+// gate/up + GeGLU + down 64 -> 38 us at 5 columns, 225 -> 46 at 21, 482 -> 73
+// at 60; the 262144-row head at 5 columns 411 -> 137 us.  hp_mid_policy.h has
+// the launches these kernels take, and both sides' times at each line.
 #include "hp_common.h"
 #include "hp_f2tile.h"
 #include "hp_gelu.h"
@@ -67,15 +68,16 @@ __device__ __forceinline__ const uint8_t *group_tiles(const uint8_t *xt, int cg,
 // down, where a wave per segment would leave most SIMDs empty) and a quarter of
 // the min chain's columns.  With no more workgroups than CUs, one wave a SIMD
 // waits on each of its own instructions, and eight waves of one class (KL = 1)
-// are faster over long rows although they unpack every header twice as often.  The waves' classes are disjoint, so neither weights nor
-// activations have a second reader in the workgroup: both go straight from
-// global memory to registers, mid_depth blocks ahead, with no stage in LDS and
-// no barrier until the chains meet (measured against activations copied
-// through a ring of LDS stages by waves of their own: the copies, 46 bytes per
-// clock and CU, bounded it).  Those loads share the CU's L1 (64 bytes and one
-// address group a clock), so what lanes share is loaded once and spread by
-// lane swaps: a row's header as one dword per lane, a column's d as one dword
-// per lane of a four-lane group.
+// are faster over long rows although they unpack every header twice as often.
+// The waves' classes are disjoint, so neither weights nor activations have a
+// second reader in the workgroup: both go straight from global memory to
+// registers, mid_depth blocks ahead, with no stage in LDS and no barrier until
+// the chains meet (measured against activations copied through a ring of LDS
+// stages by waves of their own: the copies, 46 bytes per clock and CU, bounded
+// it).  Those loads share the CU's L1 (64 bytes and one address group a clock),
+// so what lanes share is loaded once and spread by lane swaps: a row's header
+// as one dword per lane, a column's d as one dword per lane of a four-lane
+// group.
 constexpr int mid_depth(int C) { return C == 1 ? 5 : 4; }
 
 // The chains' exchange at the end: [9][16 C columns][16 rows, padded to 20]

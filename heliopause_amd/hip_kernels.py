@@ -494,9 +494,9 @@ def setInputImages(enable: bool) -> None:
 
 
 def setPrefillFolds(enable: bool) -> None:
-    """Test switch: a prefill chunk's launch folds (tiles written by their
-    producers, block-range sums added by their consumers, f16 queries);
-    default on."""
+    """Test switch: the launch folds of a prefill chunk or a draft of five
+    tokens and more (tiles written by their producers, block-range sums added
+    by their consumers, f16 queries); default on."""
     assertHipOk(lib().hp_hip_set_prefill_folds(1 if enable else 0), "setPrefillFolds")
 
 

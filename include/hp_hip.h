@@ -23,7 +23,9 @@
  * hp_hip_shutdown, so a HIP graph captured earlier never points at freed
  * memory.  Growth is refused while the stream captures (HP_ERR_ARG): a
  * captured call must follow an uncaptured call of the same shape on the
- * capturing stream.  Replaying a graph concurrently with other calls on its
+ * capturing stream.  (hp_hip_matmul_multi_device of fewer than 32 columns, or
+ * with full-range Q6_K scales, is captured without one too: on slower kernels
+ * that need no scratch.)  Replaying a graph concurrently with other calls on its
  * capture stream races on that stream's scratch.
  *
  * The host-pointer matmul entry points (hp_hip_matmul, _multi, _geglu,
@@ -248,12 +250,13 @@ int32_t hp_hip_quantize_q8_k(const float *input, size_t input_len, size_t input_
                              int8_t *qs, float *d, int16_t *bsums32);
 
 /* Matvec kernel selection (no counterpart in the reference; a tuning and
- * test hook): 0 = automatic (by column count and tile count: half-split
- * vector ALU for small projections, vector ALU for one column, the
- * bit-exact mid kernels (matrix cores, every column of the launch) from five
- * columns and from two of launches with many rows, the fast prefill kernel
- * from 64 on *_device calls), 1 = always the
- * vector-ALU kernel, 2 = the matrix-core kernel whenever its LDS fits the
+ * test hook): 0 = automatic (by column count, rows, row length and types:
+ * half-split vector ALU for small projections, vector ALU for one column,
+ * vector ALU or the matrix-core kernel for two to four, the bit-exact mid
+ * kernels (matrix cores, every column of the launch) from five columns and
+ * from two of some launches with many rows, the bit-exact prefill kernel for
+ * some host calls of hundreds of columns, the fast prefill kernel from 64
+ * columns on *_device calls), 1 = always the vector-ALU kernel, 2 = the matrix-core kernel whenever its LDS fits the
  * device, 3 = the half-split vector-ALU kernel (two lanes per row-block) for
  * up to four columns, 4 = the bit-exact prefill kernel (64-column tiles) for
  * any column count, 5 = the fast prefill kernel for any column count,
@@ -269,17 +272,19 @@ int32_t hp_hip_set_matvec_kernel(int32_t which);
 /* Pre-quantised input images inside a draft step (no counterpart in the
  * reference; a test hook): with enable != 0 (the default) the norm and GeGLU
  * launches of hp_hip_decode_layers_device at 2..8 tokens also write their
- * output as the next projection's Q8_K input, which the projection copies
- * instead of quantising; with 0 every projection quantises its f32 input
- * itself.  Both give the same bits. */
+ * output as the next projection's Q8_K input where that projection runs a
+ * vector-ALU kernel (up to four tokens under the automatic selection, or as
+ * selected), which copies it instead of quantising; with 0 every such
+ * projection quantises its f32 input itself.  Both give the same bits. */
 int32_t hp_hip_set_input_images(int32_t enable);
 
-/* Launch folds of a prefill chunk in hp_hip_decode_layers_device (no
- * counterpart in the reference; a test hook): with enable != 0 (the default)
- * the norm launches write the next projection's activation tiles, the Q/K/V,
- * O and down launches leave their block-range sums for the next launch to
- * add, the attention prologue hands the queries over rounded to f16 and the
- * attention's slice merge writes O's tiles; with 0 every projection quantises
+/* Launch folds of a draft of five tokens and more or a prefill chunk in
+ * hp_hip_decode_layers_device (no counterpart in the reference; a test hook):
+ * with enable != 0 (the default) the norm launches write the next projection's
+ * activation tiles, from nine tokens on the attention prologue hands the
+ * queries over rounded to f16 and the attention's slice merge writes O's
+ * tiles, and from 64 the Q/K/V, O and down launches leave their block-range
+ * sums for the next launch to add; with 0 every projection quantises
  * its own input and reduces its own ranges, and the queries stay f32.  Both
  * give the same bits. */
 int32_t hp_hip_set_prefill_folds(int32_t enable);
