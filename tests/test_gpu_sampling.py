@@ -44,7 +44,7 @@ def _columns(rng, cols, k, count, spread):
 
 
 @pytest.mark.parametrize("opts", OPTION_SETS, ids=[f"opt{i}" for i in range(len(OPTION_SETS))])
-@pytest.mark.parametrize("k,count", [(64, 64), (40, 40), (64, 17), (1, 1)])
+@pytest.mark.parametrize("k,count", [(64, 64), (40, 40), (64, 17), (1, 1), (6, 6), (64, 63)])
 def test_sample_device_matches_oracle(opts, k, count):
     import torch
 
