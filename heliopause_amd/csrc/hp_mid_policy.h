@@ -103,6 +103,9 @@ inline bool mfma_takes(const MidShape &l, size_t cols) {
 // one's, measured at 16 to 500 segments.
 inline bool prefill_takes(const MidShape &l, size_t cols) {
   if (!l.f16 || mid_row_waves(l)) return false;  // row waves 0.41 to 0.74
+  // class pairs for want of one type, short rows: 8192 to 131072 rows of one
+  // and two blocks 0.99 to 1.26 from 40 columns, 0.69 to 0.93 at 32
+  if (l.segs >= 2ll * l.cus && l.nb <= 2 && cols > 32) return true;
   const long long work = l.segs * (long long)cols;
   // one block 0.92 to 1.01 up to 65536 segment columns, 1.08 to 1.71 from
   // 81920; 16 segments 1.08 at 1536 columns, 1.25 at 2048
@@ -117,8 +120,17 @@ inline bool prefill_takes(const MidShape &l, size_t cols) {
   return cols >= 1536 ? l.nb >= 10 : cols >= 1024 && l.nb >= 15;
 }
 
+// Rows of one block in both types (class pairs of one block: the exchange of
+// the chains is most of the launch), many of them: 131072 rows 1.13 to 1.23 up
+// to 12 columns, 0.9 to 1.0 at 16; gate/up of 16384 in single f16 operands 1.39
+// to eight columns, 0.84 from nine.  Fewer rows 0.5 to 0.98.
+inline bool one_block_mixed(const MidShape &l, size_t cols) {
+  if (!l.q4 || !l.q6 || l.nb != 1) return false;
+  return l.pair ? l.f16 && cols <= 8 && l.segs >= 8ll * l.cus : cols < 16 && l.segs >= 32ll * l.cus;
+}
+
 inline bool mid_takes(const MidShape &l, size_t cols) {
-  if (!mid_grid_fits(l, cols)) return false;
+  if (!mid_grid_fits(l, cols) || one_block_mixed(l, cols)) return false;
   return cols >= kMidMinCols ? !mfma_takes(l, cols) : mid_takes_few(l, cols);
 }
 

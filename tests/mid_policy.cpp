@@ -60,7 +60,8 @@ void few_columns() {
       for (bool q4 : {true, false}) {
         hp::MidShape l = shape(2 * 40960, k, q4, !q4, q4);
         l.pair = true;
-        check(hp::mid_takes(l, cols) == (cols == 4 || (cols == 3 && (!q4 || k >= 2560)) || k >= (q4 ? 3840 : 2560)), "gate/up");
+        check(hp::mid_takes(l, cols) == (cols == 4 || (cols == 3 && (!q4 || k >= 2560)) || k >= (q4 ? 3840 : 2560)),
+              "gate/up");
       }
   }
   check(!hp::mid_takes(shape(262144, 2560, false, true, false), 1), "one column");
@@ -87,6 +88,13 @@ void short_rows() {
     check(hp::mid_takes(shape(8192, 512, true, false, true), cols), "Q4_K row waves, two blocks");
     check(hp::mid_takes(shape(65536, 1536, true, true, true), cols) == !to8, "mixed, six blocks");
     check(hp::mid_takes(shape(16384, 1024, true, true, true), cols), "mixed, four blocks");
+    hp::MidShape l = shape(32768, 256, true, true, false);
+    check(hp::mid_takes(l, cols), "mixed, one block, full-range");
+    l.pair = true;
+    check(hp::mid_takes(l, cols), "mixed gate/up, one block, full-range");
+    l.f16 = true;
+    check(hp::mid_takes(l, cols) == !to8, "mixed gate/up, one block");
+    check(!hp::mid_takes(shape(131072, 256, true, true, false), cols), "mixed, one block, many rows");
   }
 }
 
@@ -95,7 +103,12 @@ void short_rows() {
 void many_columns() {
   for (int nb = 1; nb <= 40; nb++)
     for (long long rows : {16, 2560, 8176})
-      for (size_t cols = 1; cols < 64; cols++) check(!hp::prefill_takes(shape(rows, 256 * nb, true, false, true), cols), "below 64");
+      for (size_t cols = 1; cols < 64; cols++)
+        check(!hp::prefill_takes(shape(rows, 256 * nb, true, false, true), cols), "below 64");
+  for (size_t cols = 30; cols < 64; cols++) {
+    check(hp::prefill_takes(shape(8192, 512, true, true, true), cols) == (cols > 32), "mixed types, short rows");
+    check(!hp::prefill_takes(shape(8192, 1024, true, true, true), cols), "mixed types, four blocks");
+  }
   check(!hp::prefill_takes(shape(2560, 256, true, false, true), 256), "one block, 40960");
   check(hp::prefill_takes(shape(2560, 256, true, false, true), 512), "one block, 81920");
   check(!hp::prefill_takes(shape(2560, 512, false, true, true), 512), "two blocks, 81920");

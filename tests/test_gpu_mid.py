@@ -155,7 +155,8 @@ def test_short_rows_of_five_to_eight_columns(hip, oracle, specs, k, m, launches)
 
 
 @pytest.mark.parametrize("specs,k,m", [
-    ([("Q4_K", 2560)], 256, 520), ([("Q6_K", 2000), ("Q4_K", 600)], 2560, 1540), ([("Q6_K", 2100)], 3840, 1030),
+    ([("Q4_K", 4100), ("Q6_K", 4100)], 256, 40), ([("Q4_K", 2560)], 256, 520),
+    ([("Q6_K", 2000), ("Q4_K", 600)], 2560, 1540), ([("Q6_K", 2100)], 3840, 1030),
 ])
 def test_many_columns_of_host_calls(hip, oracle, layouts, specs, k, m):
     """Host calls of the sizes that the bit-exact prefill kernel takes."""
@@ -282,7 +283,7 @@ def test_capture_without_scratch_leaves_no_error(hip, oracle):
 
 
 def test_failed_allocation_is_not_the_next_calls_error(hip, oracle):
-    """Every allocation of the library, scratch among them, goes through one
+    """Every device allocation of the library, scratch among them, goes through one
     function.  After one has failed (a weight of 600 GB: refused before its
     bytes are read), the launches of the next call still succeed."""
     import torch
